@@ -46,6 +46,8 @@ _SIGNATURES = {
     "fdtd_half_step_E": ([_vp, _c_i64, _vp], _c_int),
     "fdtd_half_step_H": ([_vp, _c_i64, _vp], _c_int),
     "fdtd_run": ([_vp, _c_i64, _c_i64, _vp], _c_int),
+    "fdtd_plan_step_workspace": ([_vp, _pi64], _c_int),
+    "fdtd_plan_set_step_workspace": ([_vp, _vp, _c_i64], _c_int),
     "fdtd_check_finite": ([_vp, _vp, _vp], _c_int),
     "fdtd_bench_main_kernel": ([_vp, _c_i64, _vp, ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_float)],
                                _c_int),
@@ -147,6 +149,7 @@ class Plan:
                                  E.data_ptr(), H.data_ptr(), inv_eps.data_ptr(), inv_mu.data_ptr(),
                                  ctypes.byref(h)))
         self._h = h
+        self.step_buf = None  # whole-step workspace: None not asked for yet, False none
         self._keep = [E, H, inv_eps, inv_mu]
         if pitch is not None and pitch != shape[1] * shape[2]:
             check(L.fdtd_plan_set_pitch(h, int(pitch)))
@@ -223,6 +226,17 @@ class Plan:
 
     def run(self, q0, nsteps, stream):
         check(self._L.fdtd_run(self._h, q0, nsteps, stream))
+
+    def step_workspace(self):
+        """Bytes of the whole-step workspace; 0 when the plan has no use for one."""
+        n = ctypes.c_int64()
+        check(self._L.fdtd_plan_step_workspace(self._h, ctypes.byref(n)))
+        return n.value
+
+    def set_step_workspace(self, buf):
+        """Lend the uint8 device tensor `buf` to the plan's whole steps."""
+        check(self._L.fdtd_plan_set_step_workspace(self._h, buf.data_ptr(), buf.numel()))
+        self.step_buf = buf
 
     def check_finite(self, flag, stream):
         """OR 1 into the device int32 tensor `flag` if an E or H value is

@@ -8,12 +8,15 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "fdtd_hip.h"
 #include "fdtd_kernels.hpp"
+#include "fdtd_step.hpp"
 
 using namespace fdtd_dev;
 
@@ -128,6 +131,19 @@ struct FdtdPlan {
   void* rec_curl = nullptr;
   void* rec_plane = nullptr;
   Box rec_db{}, rec_pb{};
+  // whole-step kernel (fdtd_plan_set_step_workspace): the caller's workspace
+  // holds a second E, H and psiE; the device tables below belong to the plan
+  void* step_ws = nullptr;
+  void* step_dev = nullptr;
+  StepSide* d_sides[2] = {nullptr, nullptr};  // E -> second E, and back
+  StepSrc* d_ssrcs = nullptr;
+  StepDet* d_sdets = nullptr;
+  struct StepTile {
+    int tx, ty, tz, ntx, nty, ntz;
+  } step_tile{};
+  int step_order = 0;  // StepArgs::order
+  CopySeg* d_back = nullptr;  // workspace -> plan, after an odd last step
+  int nback = 0;
 };
 
 struct FdtdBatch {
@@ -208,6 +224,20 @@ void free_tables(FdtdPlan* p) {
   p->d_curs = nullptr;
 }
 
+// Forgets the whole-step workspace (the tables point into it and into the
+// plan's arrays).
+void free_step(FdtdPlan* p) {
+  if (p->step_dev) {
+    (void)hipDeviceSynchronize();
+    (void)hipFree(p->step_dev);
+  }
+  p->step_dev = nullptr;
+  p->step_ws = nullptr;
+  p->d_sides[0] = p->d_sides[1] = nullptr;
+  p->d_ssrcs = nullptr;
+  p->d_sdets = nullptr;
+}
+
 int select_device(const FdtdPlan* p) {
   int cur = -1;
   FDTD_HIP(hipGetDevice(&cur));
@@ -217,26 +247,12 @@ int select_device(const FdtdPlan* p) {
 
 // Field and material policies of a plan (see fdtd_kernels.hpp).
 template <class FS>
-FS make_field(const FdtdPlan* p, bool H);
-template <>
-PlainField<double, double> make_field(const FdtdPlan* p, bool H) {
-  return {reinterpret_cast<double*>(H ? p->H : p->E), p->d.cs};
+FS field_at(void* p, int64_t cs) {
+  return {static_cast<typename FS::Elem*>(p), cs};
 }
-template <>
-PlainField<float, float> make_field(const FdtdPlan* p, bool H) {
-  return {reinterpret_cast<float*>(H ? p->H : p->E), p->d.cs};
-}
-template <>
-CompField make_field(const FdtdPlan* p, bool H) {
-  return {reinterpret_cast<float*>(H ? p->H : p->E), p->d.cs};
-}
-template <>
-PlainField<cplx<double>, cplx<double>> make_field(const FdtdPlan* p, bool H) {
-  return {reinterpret_cast<cplx<double>*>(H ? p->H : p->E), p->d.cs};
-}
-template <>
-PlainField<cplx<float>, cplx<float>> make_field(const FdtdPlan* p, bool H) {
-  return {reinterpret_cast<cplx<float>*>(H ? p->H : p->E), p->d.cs};
+template <class FS>
+FS make_field(const FdtdPlan* p, bool H) {
+  return field_at<FS>(H ? p->H : p->E, p->d.cs);
 }
 template <class MS>
 MS make_mat(const FdtdPlan* p, bool mu);
@@ -444,6 +460,308 @@ int check_step_room(const FdtdPlan* p, int64_t q0, int64_t nsteps, bool is_H_onl
 
 int half_dispatch(FdtdPlan* p, bool is_H, int64_t q, hipStream_t st) {
   return with_policies(p, [&]<class FS, class MS, typename O>() { return launch_half<FS, MS, O>(p, is_H, q, st); });
+}
+
+// ------------------------------------------------------------- whole steps
+size_t value_bytes(const FdtdPlan* p) {  // bytes of a CPML value (the arithmetic type)
+  switch (p->dtype) {
+    case FDTD_F32: return 4;
+    case FDTD_C128: return 16;
+    default: return 8;  // F64, F32C (float64 CPML state), C64
+  }
+}
+size_t field_bytes(const FdtdPlan* p) {  // one field array
+  return (p->dtype == FDTD_F32C ? (size_t)4 * sizeof(float) : 3 * value_bytes(p)) * (size_t)p->d.cs;
+}
+
+// Cells in ascending order; false when a cell occurs twice.
+bool sorted_cells(const std::vector<int64_t>& cells, std::vector<int32_t>& order) {
+  order.resize(cells.size());
+  for (size_t i = 0; i < cells.size(); ++i) order[i] = (int32_t)i;
+  if (std::adjacent_find(cells.begin(), cells.end(), std::greater_equal<int64_t>()) == cells.end()) return true;
+  std::sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return cells[a] < cells[b]; });
+  for (size_t i = 1; i < order.size(); ++i)
+    if (cells[order[i]] == cells[order[i - 1]]) return false;
+  return true;
+}
+
+Box cells_box(const FdtdPlan* p, const std::vector<int64_t>& cells) {
+  Box b{INT32_MAX, 0, INT32_MAX, 0, INT32_MAX, 0};
+  for (int64_t c : cells) {
+    const int32_t i = (int32_t)(c / p->d.px), r = (int32_t)(c % p->d.px), j = r / p->d.nz, k = r % p->d.nz;
+    b = Box{std::min(b.x0, i), std::max(b.x1, i + 1), std::min(b.y0, j),
+            std::max(b.y1, j + 1), std::min(b.z0, k), std::max(b.z1, k + 1)};
+  }
+  return b;
+}
+
+// The order in which a cell's faces along the three axes are applied, as
+// StepArgs::order, or -1 when no one order holds for every combination of
+// sides (the order is the faces' registration order), or when a side has
+// several faces or the two slabs of an axis overlap.
+int face_order(const FdtdPlan* p) {
+  int rank[3][2], t[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  for (size_t f = 0; f < p->faces.size(); ++f) {
+    const FaceHost& fh = p->faces[f];
+    if (t[fh.axis][fh.high]) return -1;
+    t[fh.axis][fh.high] = fh.t;
+    rank[fh.axis][fh.high] = (int)f;
+  }
+  const int n[3] = {p->d.nx, p->d.ny, p->d.nz};
+  for (int ax = 0; ax < 3; ++ax)
+    if (t[ax][0] + t[ax][1] > n[ax]) return -1;
+  // whether every face along a comes before every face along b
+  auto before = [&](int a, int b) {
+    for (int u = 0; u < 2; ++u)
+      for (int v = 0; v < 2; ++v)
+        if (t[a][u] && t[b][v] && rank[a][u] > rank[b][v]) return false;
+    return true;
+  };
+  int ax[3] = {0, 1, 2};
+  do {
+    if (before(ax[0], ax[1]) && before(ax[0], ax[2]) && before(ax[1], ax[2])) return ax[0] | ax[1] << 2 | ax[2] << 4;
+  } while (std::next_permutation(ax, ax + 3));
+  return -1;
+}
+
+// Whether the plan's whole step can run as one kernel: nothing but the E half
+// step's own update may stand between a cell's E and the H that reads it. A
+// periodic copy (of an axis longer than one cell) and a soft source, which
+// reads a current measured on the finished H, do stand there.
+//
+// A whole step saves launches and the second pass over the fields and pays
+// with the halo cells on which neighbouring workgroups compute the same E
+// (40-60 % of the work-items of a 3D tile, 10-15 % of a 2D one). Up to which
+// size that pays, measured on MI355X against the half steps (us/step, half
+// steps -> whole): 2D 161x97 float64 16.3 -> 5.9, 1400x1400 103 -> 86 (2000 x
+// 2000 173 -> 174); 3D float64 60x52x44 21.0 -> 14.3, 110^3 67.9 -> 60.4 (128^3
+// 92 -> 132); float32 36^3 11.1 -> 7.0, 56^3 12.4 -> 12.0 (72^3 15.1 -> 17.0);
+// compensated 40^3 11.9 -> 8.2, 100^3 42.8 -> 39.5. Complex values take twice the
+// registers and lose from 48^3 on (complex64 from 32^3): half steps only.
+// FDTD_HIP_STEP: 0 never, 1 whatever the size (the rest of the rule stands).
+bool step_eligible(const FdtdPlan* p) {
+  if (is_complex(p)) return false;
+  const bool flat = p->d.nx == 1 || p->d.ny == 1 || p->d.nz == 1;
+  const int64_t most = (int64_t)1 << (flat ? 21 : (p->dtype == FDTD_F32 ? 17 : 20));
+  const char* env = getenv("FDTD_HIP_STEP");
+  if (env ? atoi(env) == 0 : grid_cells(p) > most) return false;
+  if (face_order(p) < 0 || p->srcs.size() > 32 || p->dets.size() > 32 || !p->curs.empty()) return false;
+  if (p->d.cs >= (int64_t)1 << 28) return false;  // 32-bit byte offsets
+  for (const Bnd& b : p->stages) {
+    const int n = b.index == 0 ? p->d.nx : (b.index == 1 ? p->d.ny : p->d.nz);
+    if (b.periodic ? n > 1 : p->dtype == FDTD_F32C) return false;
+  }
+  // 32-bit byte offsets into a component of a face's psi
+  for (const FaceHost& f : p->faces)
+    if ((size_t)(plane_cells(p, f.axis) * f.t) * value_bytes(p) >= (size_t)1 << 32) return false;
+  std::vector<int32_t> order;
+  for (const SrcHost& s : p->srcs)
+    if (s.kind == FDTD_SRC_SOFT || !sorted_cells(s.cells, order)) return false;
+  for (const DetHost& dh : p->dets)
+    if (!sorted_cells(dh.cells, order)) return false;
+  return true;
+}
+
+size_t step_workspace(const FdtdPlan* p) {
+  size_t n = 2 * align_up(field_bytes(p));
+  for (const FaceHost& f : p->faces) n += align_up(2 * (size_t)(plane_cells(p, f.axis) * f.t) * value_bytes(p));
+  return n;
+}
+
+// Tile of the whole-step kernel: the shape with the fewest workgroups over the
+// grid, rows of z cells as long as a cache line where there is a choice.
+void step_shape(const FdtdPlan* p, FdtdPlan::StepTile& best) {
+  const Dims& d = p->d;
+  constexpr int threads = kStepThreads;
+  double cost = 1e30;
+  for (int tz = 1; tz <= std::min(d.nz, threads); ++tz)
+    for (int ty = 1; ty <= std::min(d.ny, threads / tz); ++ty) {
+      // most x planes whose own and halo cells fit (an axis with one tile has no halo)
+      const int hy = ty < d.ny ? tz : 0, hz = tz < d.nz ? ty : 0;
+      int tx = threads / (ty * tz + hy + hz);
+      if (tx < d.nx) tx = (threads - ty * tz) / (ty * tz + hy + hz);
+      tx = std::min(tx, d.nx);
+      if (tx < 1) continue;
+      const int ntx = (d.nx + tx - 1) / tx, nty = (d.ny + ty - 1) / ty, ntz = (d.nz + tz - 1) / tz;
+      const double c = (double)ntx * nty * ntz * (1.0 + 4.0 / std::min(tz, 64));
+      if (c < cost) {
+        cost = c;
+        best = {tx, ty, tz, ntx, nty, ntz};
+      }
+    }
+}
+
+// Device tables of the whole step for the workspace p->step_ws.
+int build_step_tables(FdtdPlan* p) {
+  const size_t nf = p->faces.size(), ns = p->srcs.size(), nd = p->dets.size();
+  size_t off = 0;
+  auto take = [&](size_t n) {
+    const size_t at = off;
+    off = align_up(off + n);
+    return at;
+  };
+  const size_t o_f[2] = {take(6 * sizeof(StepSide)), take(6 * sizeof(StepSide))};
+  const size_t o_s = take(ns * sizeof(StepSrc)), o_d = take(nd * sizeof(StepDet)), o_b = take((2 + nf) * sizeof(CopySeg));
+  std::vector<size_t> o_sc(ns), o_sp(ns), o_dc(nd), o_do(nd);
+  for (size_t i = 0; i < ns; ++i) {
+    o_sc[i] = take(p->srcs[i].cells.size() * sizeof(int64_t));
+    o_sp[i] = take(p->srcs[i].profile.size() * sizeof(double));
+  }
+  for (size_t i = 0; i < nd; ++i) {
+    o_dc[i] = take(p->dets[i].cells.size() * sizeof(int64_t));
+    o_do[i] = take(p->dets[i].cells.size() * sizeof(int32_t));
+  }
+  const size_t total = off > 0 ? off : 256;
+  std::vector<unsigned char> host(total, 0);
+  FDTD_HIP(hipMalloc(&p->step_dev, total));
+  char* base = reinterpret_cast<char*>(p->step_dev);
+  char* const ws = reinterpret_cast<char*>(p->step_ws);
+  char* psi2 = ws + 2 * align_up(field_bytes(p));
+  std::vector<CopySeg> back;
+  auto copy_back = [&](const void* src, void* dst, size_t bytes) {
+    back.push_back({static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), (int64_t)(bytes / 4)});
+  };
+  copy_back(ws, p->E, field_bytes(p));
+  copy_back(ws + align_up(field_bytes(p)), p->H, field_bytes(p));
+  for (size_t i = 0; i < nf; ++i) {
+    const FaceDev& fd = p->h_faces[i];
+    const size_t at = (size_t)(fd.axis * 2 + (fd.high ? 1 : 0)) * sizeof(StepSide);
+    const size_t comp = (size_t)fd.slab * value_bytes(p);
+    char *psiE = static_cast<char*>(fd.psiE), *psiH = static_cast<char*>(fd.psiH);
+    StepSide sd{{psiE, psiE + comp}, {psi2, psi2 + comp}, {psiH, psiH + comp}, fd.bE, fd.cE, fd.bH, fd.cH};
+    std::memcpy(host.data() + o_f[0] + at, &sd, sizeof(sd));
+    for (int c = 0; c < 2; ++c) {
+      sd.psiE_in[c] = psi2 + c * comp;
+      sd.psiE_out[c] = psiE + c * comp;
+    }
+    std::memcpy(host.data() + o_f[1] + at, &sd, sizeof(sd));
+    copy_back(psi2, psiE, 2 * comp);
+    psi2 += align_up(2 * (size_t)fd.slab * value_bytes(p));
+  }
+  std::memcpy(host.data() + o_b, back.data(), back.size() * sizeof(CopySeg));
+  std::vector<int32_t> order;
+  for (size_t i = 0; i < ns; ++i) {
+    const SrcHost& s = p->srcs[i];
+    sorted_cells(s.cells, order);
+    StepSrc ss{};
+    ss.kind = s.kind;
+    ss.compE = s.compE;
+    ss.compH = s.compH;
+    ss.n = (int32_t)s.cells.size();
+    ss.box = cells_box(p, s.cells);
+    ss.dense = box_cells(ss.box) == ss.n;
+    ss.cells = reinterpret_cast<const int64_t*>(base + o_sc[i]);
+    ss.profile = reinterpret_cast<const double*>(base + o_sp[i]);
+    ss.amplitude = s.amplitude;
+    for (size_t c = 0; c < order.size(); ++c) {
+      std::memcpy(host.data() + o_sc[i] + c * 8, &s.cells[order[c]], 8);
+      if (!s.profile.empty()) std::memcpy(host.data() + o_sp[i] + c * 8, &s.profile[order[c]], 8);
+    }
+    std::memcpy(host.data() + o_s + i * sizeof(ss), &ss, sizeof(ss));
+  }
+  for (size_t i = 0; i < nd; ++i) {
+    const DetHost& dh = p->dets[i];
+    sorted_cells(dh.cells, order);
+    StepDet sd{};
+    sd.n = (int32_t)dh.cells.size();
+    sd.box = cells_box(p, dh.cells);
+    sd.dense = box_cells(sd.box) == sd.n;
+    sd.cells = reinterpret_cast<const int64_t*>(base + o_dc[i]);
+    sd.order = reinterpret_cast<const int32_t*>(base + o_do[i]);
+    sd.bufE = dh.bufE;
+    sd.bufH = dh.bufH;
+    sd.slot0E = p->nE - dh.countE;
+    sd.slot0H = p->nH - dh.countH;
+    for (size_t c = 0; c < order.size(); ++c) std::memcpy(host.data() + o_dc[i] + c * 8, &dh.cells[order[c]], 8);
+    std::memcpy(host.data() + o_do[i], order.data(), order.size() * 4);
+    std::memcpy(host.data() + o_d + i * sizeof(sd), &sd, sizeof(sd));
+  }
+  step_shape(p, p->step_tile);
+  p->step_order = face_order(p);
+  FDTD_HIP(hipMemcpy(p->step_dev, host.data(), total, hipMemcpyHostToDevice));
+  for (int h = 0; h < 2; ++h) p->d_sides[h] = reinterpret_cast<StepSide*>(base + o_f[h]);
+  p->d_back = reinterpret_cast<CopySeg*>(base + o_b);
+  p->nback = (int)back.size();
+  p->d_ssrcs = reinterpret_cast<StepSrc*>(base + o_s);
+  p->d_sdets = reinterpret_cast<StepDet*>(base + o_d);
+  return 0;
+}
+
+// One whole step; `back`: from the workspace's fields into the plan's.
+template <class FS, class MS, typename O>
+int launch_step(FdtdPlan* p, bool back, int64_t q, hipStream_t st) {
+  if constexpr (std::is_same_v<typename FS::R, cplx<double>> || std::is_same_v<typename FS::R, cplx<float>>) {
+    return fail(-1, "no whole steps on complex fields");  // step_eligible: not reached
+  } else {
+    StepArgs<FS, MS> a{};
+    char* const ws = static_cast<char*>(p->step_ws);
+    const FS E = make_field<FS>(p, false), H = make_field<FS>(p, true), E2 = field_at<FS>(ws, p->d.cs),
+             H2 = field_at<FS>(ws + align_up(field_bytes(p)), p->d.cs);
+    a.d = p->d;
+    a.sc = (typename FS::R)p->sc;
+    a.E = back ? E2 : E;
+    a.H = back ? H2 : H;
+    a.E2 = back ? E : E2;
+    a.H2 = back ? H : H2;
+    a.Me = make_mat<MS>(p, false);
+    a.Mu = make_mat<MS>(p, true);
+    a.sides = p->d_sides[back ? 1 : 0];
+    for (const FaceHost& f : p->faces) a.t[f.axis * 2 + f.high] = f.t;
+    a.order = p->step_order;
+    a.objs = p->d_objs;
+    a.nobjs = (int32_t)p->objs.size();
+    a.srcs = p->d_ssrcs;
+    a.nsrc = (int32_t)p->srcs.size();
+    a.dets = p->d_sdets;
+    a.ndet = (int32_t)p->dets.size();
+    a.folded = p->fold_points;
+    a.wave = p->wave;
+    a.wave_cap = p->wave_cap;
+    a.q = q;
+    a.nE = p->nE;
+    a.nH = p->nH;
+    const FdtdPlan::StepTile& t = p->step_tile;
+    a.tx = t.tx;
+    a.ty = t.ty;
+    a.tz = t.tz;
+    a.ntx = t.ntx;
+    a.nty = t.nty;
+    a.ntz = t.ntz;
+    const dim3 g((unsigned)(t.ntx * t.nty * t.ntz)), b(kStepThreads);
+    if (a.nobjs)
+      hipLaunchKernelGGL((k_step<FS, MS, O, true>), g, b, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_step<FS, MS, O, false>), g, b, 0, st, a);
+    FDTD_HIP(hipGetLastError());
+    ++p->nE;
+    ++p->nH;
+    for (DetHost& dh : p->dets) ++dh.countE, ++dh.countH;
+    return 0;
+  }
+}
+
+int step_dispatch(FdtdPlan* p, bool back, int64_t q, hipStream_t st) {
+  return with_policies(p, [&]<class FS, class MS, typename O>() { return launch_step<FS, MS, O>(p, back, q, st); });
+}
+
+// nsteps steps from time index q0: with a workspace as whole steps, out to the
+// second fields and back (an odd last one is copied back), else half by half
+// in place.
+int run_steps(FdtdPlan* p, int64_t q0, int64_t nsteps, hipStream_t st) {
+  if (!p->step_ws) {
+    for (int64_t s = 0; s < nsteps; ++s) {
+      if (int rc = half_dispatch(p, false, q0 + s, st)) return rc;
+      if (int rc = half_dispatch(p, true, q0 + s, st)) return rc;
+    }
+    return 0;
+  }
+  for (int64_t s = 0; s < nsteps; ++s)
+    if (int rc = step_dispatch(p, s % 2 == 1, q0 + s, st)) return rc;
+  if (nsteps % 2 == 0) return 0;
+  const int64_t blocks = std::min<int64_t>((int64_t)(field_bytes(p) / 4 + 1023) / 1024, 1024);
+  hipLaunchKernelGGL(k_copy_back, dim3((unsigned)blocks), dim3(256), 0, st, (const CopySeg*)p->d_back, p->nback);
+  FDTD_HIP(hipGetLastError());
+  return 0;
 }
 
 int adj_check_plan(const FdtdPlan* p) {
@@ -917,6 +1235,7 @@ int fdtd_plan_create(int dtype, int nx, int ny, int nz, double courant_number, v
 
 int fdtd_plan_destroy(FdtdPlan* plan) {
   if (!plan) return 0;
+  free_step(plan);
   free_tables(plan);
   delete plan;
   return 0;
@@ -1128,6 +1447,7 @@ int fdtd_plan_finalize(FdtdPlan* p) {
   if (!p) return fail(-1, "null plan");
   if (p->dtype == FDTD_F32C && (!p->E_lo || !p->H_lo)) return fail(-1, "FDTD_F32C plan without compensation arrays");
   if (int rc = select_device(p)) return rc;
+  free_step(p);
   free_tables(p);
   // boundaries before the first periodic one fold into the main kernels
   p->n_fused = 0;
@@ -1335,9 +1655,28 @@ int fdtd_run(FdtdPlan* p, int64_t q0, int64_t nsteps, void* stream) {
   if (int rc = check_step_room(p, q0, nsteps, false, false)) return rc;
   if (int rc = select_device(p)) return rc;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  for (int64_t s = 0; s < nsteps; ++s) {
-    if (int rc = half_dispatch(p, false, q0 + s, st)) return rc;
-    if (int rc = half_dispatch(p, true, q0 + s, st)) return rc;
+  return run_steps(p, q0, nsteps, st);
+}
+
+int fdtd_plan_step_workspace(const FdtdPlan* p, int64_t* bytes) {
+  if (int rc = check_plan(p)) return rc;
+  if (!bytes) return fail(-1, "null argument");
+  *bytes = step_eligible(p) ? (int64_t)step_workspace(p) : 0;
+  return 0;
+}
+
+int fdtd_plan_set_step_workspace(FdtdPlan* p, void* workspace, int64_t bytes) {
+  if (int rc = check_plan(p)) return rc;
+  if (int rc = select_device(p)) return rc;
+  free_step(p);
+  if (!workspace) return 0;
+  if (!step_eligible(p)) return fail(-1, "this plan's steps do not run as one kernel");
+  if (bytes < (int64_t)step_workspace(p)) return fail(-1, "step workspace too small");
+  if (reinterpret_cast<uintptr_t>(workspace) & 15) return fail(-1, "the step workspace must be 16-byte aligned");
+  p->step_ws = workspace;
+  if (int rc = build_step_tables(p)) {
+    free_step(p);
+    return rc;
   }
   return 0;
 }

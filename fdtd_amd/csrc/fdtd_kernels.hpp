@@ -127,6 +127,17 @@ __device__ __forceinline__ gptr<T> gp(T* p) {
   return (gptr<T>)p;
 }
 
+// p[0] of an array whose base is the same for the whole wavefront, `off` bytes
+// further on.
+template <typename T>
+__device__ __forceinline__ T* split_ptr(T* p, uint32_t off) {
+  return (T*)((gptr<char>)gp(p) + off);
+}
+template <typename T>
+__device__ __forceinline__ const T* split_ptr(const T* p, uint32_t off) {
+  return (const T*)((gptr<const char>)gp(p) + off);
+}
+
 template <bool NT, typename T>
 __device__ __forceinline__ T ld_stream(const T* p) {
   if constexpr (NT) return __builtin_nontemporal_load(gp(p));
@@ -195,6 +206,7 @@ template <typename S, typename R_>
 struct PlainField {
   using R = R_;
   using Sample = S;
+  using Elem = S;
   static constexpr bool kRecords = false;  // the marching kernels' record path (CompField) is off
   struct Rec {};
   S* p;
@@ -219,6 +231,38 @@ struct PlainField {
   __device__ __forceinline__ void put(int64_t i, R v) const { st_stream<false>(p + i, (S)v); }
   __device__ __forceinline__ void copy(int64_t dst, int64_t src) const { st_stream<false>(p + dst, ld_stream<false>(p + src)); }
   __device__ __forceinline__ Sample sample(int64_t i) const { return ld_stream<false>(p + i); }
+  // The same accesses with the cell split into a part that is the same for
+  // the whole wavefront and a byte offset of 32 bits per work-item, which is
+  // the form a global access takes without any address arithmetic. Own: the
+  // three components of a cell, Duo: two of a neighbour's, as loaded.
+  static constexpr uint32_t kCell = sizeof(S);
+  struct Own {
+    S v[3];
+  };
+  struct Duo {
+    S a, b;
+  };
+  __device__ __forceinline__ S* at(int c, int64_t uni, uint32_t off) const { return split_ptr(p + c * cs + uni, off); }
+  template <bool NT>
+  __device__ __forceinline__ Own own(int64_t uni, uint32_t off) const {
+    return {{ld_stream<NT>(at(0, uni, off)), ld_stream<NT>(at(1, uni, off)), ld_stream<NT>(at(2, uni, off))}};
+  }
+  template <int C0, int C1>
+  __device__ __forceinline__ Duo duo(int64_t uni, uint32_t off) const {
+    return {ld_stream<false>(at(C0, uni, off)), ld_stream<false>(at(C1, uni, off))};
+  }
+  template <int C>
+  static __device__ __forceinline__ R value(const Own& o) { return (R)o.v[C]; }
+  template <int C0, int C1, int C>
+  static __device__ __forceinline__ R value(const Duo& o) { return (R)(C == C0 ? o.a : o.b); }
+  template <bool NT>
+  __device__ __forceinline__ void put_own(int64_t uni, uint32_t off, const R v[3]) const {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) st_stream<NT>(at(c, uni, off), (S)v[c]);
+  }
+  // the value as a store and a load leave it, and as a detector samples it
+  static __device__ __forceinline__ R rounded(R v) { return v; }
+  static __device__ __forceinline__ Sample sampled(R v) { return (S)v; }
 };
 
 // Compensated storage: a value v is kept as the float h holding the top 24
@@ -260,6 +304,7 @@ typedef float f32x4 __attribute__((vector_size(16)));
 struct CompField {
   using R = double;
   using Sample = float;
+  using Elem = float;
   // The marching kernels keep the previous plane's record as loaded and
   // decode it where it is used: a decoded carry is computed right after its
   // load, ahead of the branch that guards a cell's store, so the wave would
@@ -298,6 +343,40 @@ struct CompField {
   }
   // detectors sample the value rounded to float
   __device__ __forceinline__ float sample(int64_t i) const { return (float)get(i); }
+  static constexpr uint32_t kCell = 16;
+  using Own = f32x4;
+  using Duo = f32x4;
+  template <bool NT>
+  __device__ __forceinline__ Own own(int64_t uni, uint32_t off) const {
+    return ld_stream<NT>(split_ptr(reinterpret_cast<const f32x4*>(rec) + uni, off));
+  }
+  template <int C0, int C1>
+  __device__ __forceinline__ Duo duo(int64_t uni, uint32_t off) const { return own<false>(uni, off); }
+  template <int C>
+  static __device__ __forceinline__ double value(const f32x4& r) { return decode_c<C>(r); }
+  template <int C0, int C1, int C>
+  static __device__ __forceinline__ double value(const f32x4& r) { return decode_c<C>(r); }
+  template <bool NT>
+  __device__ __forceinline__ void put_own(int64_t uni, uint32_t off, const double v[3]) const {
+    f32x4 r;
+    uint32_t w = 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      uint32_t q;
+      r[c] = comp_hi(v[c], q);
+      w |= q << (8 * c);
+    }
+    r[3] = __uint_as_float(w);
+    float* const at = split_ptr(rec + 4 * uni, off);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) st_stream<NT>(at + c, (float)r[c]);
+  }
+  static __device__ __forceinline__ double rounded(double v) {
+    uint32_t q;
+    const float h = comp_hi(v, q);
+    return comp_decode(h, q);
+  }
+  static __device__ __forceinline__ float sampled(double v) { return (float)rounded(v); }
   __device__ __forceinline__ Rec rec3(int64_t cell) const { return record<false>(cell); }
   template <int C>
   static __device__ __forceinline__ double decode_c(const f32x4& r) {
@@ -349,6 +428,20 @@ struct MatArray {
 #pragma unroll
     for (int c = 0; c < 3; ++c) m[c] = (R)ld_stream<NT>(p + c * cs + i);
   }
+  // as PlainField's: what is loaded for a cell, and its three values
+  static constexpr uint32_t kCell = sizeof(S);
+  struct Own {
+    S v[3];
+  };
+  template <bool NT>
+  __device__ __forceinline__ Own own(int64_t uni, uint32_t off) const {
+    return {{ld_stream<NT>(split_ptr(p + uni, off)), ld_stream<NT>(split_ptr(p + cs + uni, off)),
+             ld_stream<NT>(split_ptr(p + 2 * cs + uni, off))}};
+  }
+  __device__ __forceinline__ void values(const Own& o, R m[3]) const {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) m[c] = (R)o.v[c];
+  }
 };
 
 template <typename R>
@@ -362,6 +455,15 @@ struct MatPalette {
   __device__ __forceinline__ void get3(Key k, int64_t, R m[3]) const {
 #pragma unroll
     for (int c = 0; c < 3; ++c) m[c] = (R)gp(tab)[3 * k + c];
+  }
+  static constexpr uint32_t kCell = 1;
+  using Own = uint8_t;
+  template <bool NT>
+  __device__ __forceinline__ Own own(int64_t uni, uint32_t off) const { return ld_stream<NT>(split_ptr(id + uni, off)); }
+  __device__ __forceinline__ void values(const Own& o, R m[3]) const {
+    const uint32_t at = 3 * sizeof(double) * o;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) m[c] = (R)ld_stream<false>(split_ptr(tab + c, at));
   }
 };
 

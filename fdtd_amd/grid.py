@@ -141,6 +141,7 @@ class Grid:
         self._plan_key = None
         self._wave = None
         self._wave_key = None
+        self._step_buf = None
 
     # ------------------------------------------------------------ storage
     def _alloc_soa(self, dtype):
@@ -437,6 +438,30 @@ class Grid:
         self._wave_key = key
         self._plan.set_waveforms(self._wave)
 
+    def _lend_step_workspace(self, plan):
+        """Give `plan` the memory for a second copy of the fields, with which
+        it takes a step as one kernel (small grids); without room for it the
+        plan goes on stepping half by half, in place."""
+        cuda = self._E.is_cuda
+        if plan.step_buf is None:
+            if cuda and torch.cuda.is_current_stream_capturing():
+                return  # the plan's tables cannot be built in a capture
+            plan.step_buf = False
+            need = plan.step_workspace()
+            if need == 0:
+                self._step_buf = None
+                return
+            if self._step_buf is None or self._step_buf.numel() < need:
+                try:
+                    self._step_buf = torch.empty(need, dtype=torch.uint8, device=self._E.device)
+                except torch.cuda.OutOfMemoryError:
+                    self._step_buf = None
+                    return
+                self._step_stream = torch.cuda.current_stream() if cuda else None
+            plan.set_step_workspace(self._step_buf)
+        if cuda and plan.step_buf is not False and torch.cuda.current_stream() != self._step_stream:
+            plan.step_buf.record_stream(torch.cuda.current_stream())
+
     def _prepare(self, nsteps, e_steps, h_steps):
         plan = self._ensure_plan()
         grown = False
@@ -480,10 +505,11 @@ class Grid:
         if progress_bar:
             from tqdm import tqdm
             bar = tqdm(total=n)
-            per = max(1, n // 100)
+            per = max(2, n // 100)  # whole steps go in pairs
             chunks = [per] * (n // per) + ([n % per] if n % per else [])
         for m in chunks:
             plan = self._prepare(m, m, m)
+            self._lend_step_workspace(plan)
             plan.run(self.time_steps_passed, m, self._stream())
             self._count_halves(m, m)
             self.time_steps_passed += m

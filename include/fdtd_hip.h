@@ -186,6 +186,20 @@ int fdtd_half_step_H(FdtdPlan* plan, int64_t q, void* stream);
  * E half step then H half step at q, then q+1. */
 int fdtd_run(FdtdPlan* plan, int64_t q0, int64_t nsteps, void* stream);
 
+/* Optional, after fdtd_plan_finalize: device memory in which fdtd_run keeps a
+ * second copy of the fields, so that it can take each step as one kernel
+ * (the two half steps in one sweep, from the plan's arrays to the copy and
+ * back; the results are the half steps' own, bit for bit, and after every
+ * call they are in the plan's arrays). fdtd_plan_step_workspace gives its
+ * size in bytes, 0 for a plan whose half steps cannot be joined (a periodic
+ * boundary along an axis of several cells, a soft source or a current
+ * detector, a source or detector with a cell named twice). The workspace is
+ * 16-byte aligned, borrowed until fdtd_plan_destroy, the next
+ * fdtd_plan_finalize or a call with NULL, and holds nothing between calls.
+ * No counterpart in the reference. */
+int fdtd_plan_step_workspace(const FdtdPlan* plan, int64_t* bytes);
+int fdtd_plan_set_step_workspace(FdtdPlan* plan, void* workspace, int64_t bytes);
+
 /* No counterpart in the reference, whose only guard against divergence is
  * the Courant limit at construction (fdtd/grid.py:123-127): launch on
  * `stream` a check of every E and H value of the plan and OR 1 into the

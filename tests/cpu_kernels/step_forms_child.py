@@ -1,0 +1,25 @@
+"""Child process of tests/test_whole_step.py: every form of tests/step_forms.py
+on the host copy of the kernels (see replay.py), one JSON line per form."""
+
+import json
+import os
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, HERE)
+sys.path.insert(0, os.path.dirname(HERE))
+
+import replay  # noqa: E402
+import step_forms  # noqa: E402
+
+
+def main():
+    replay.load()
+    for arg in sys.argv[1:]:
+        name, backend = arg.split("/")
+        bad = step_forms.differences(replay.fdtd, name, backend)
+        print(json.dumps({"form": arg, "bad": bad}), flush=True)
+
+
+if __name__ == "__main__":
+    main()

@@ -1,0 +1,138 @@
+"""Grids whose ``run`` may take whole steps (one kernel a step), and a
+comparison of such a run with the same run taken half step by half step
+(FDTD_HIP_STEP=0): every field, CPML and trace value must have the same bits.
+
+The forms cover the whole-step rule and its edges: flat and 3D grids smaller
+than a tile, of one cell more than a tile, and of many tiles with remainders;
+CPML on any side, of any thickness, in any registration order (orders that
+differ between sides, and slabs that overlap, go half by half); every object
+kind; folded and unfolded point sources, straight, diagonal and list lines,
+plane sources; line, diagonal and block detectors (sources or detectors that
+name a cell twice go half by half).
+"""
+
+import os
+
+import numpy as np
+import torch
+
+S = slice
+FULL = (S(None), S(None), S(None))
+
+
+def face(axis, high, t):
+    key = list(FULL)
+    key[axis] = S(-t, None) if high else S(0, t)
+    return ("PML", {}, tuple(key))
+
+
+def faces(t, axes=(0, 1, 2)):
+    return [face(a, h, t) for a in axes for h in (0, 1)]
+
+
+POINT = ("PointSource", dict(period=9, amplitude=0.7), "mid")
+FORMS = {
+    # name: (shape, components, whether whole steps are taken)
+    "one_cell_rows": ((37, 1, 1), [face(0, 0, 4), face(0, 1, 3), POINT], True),
+    "flat_z": ((23, 41, 1), faces(5, (0, 1)) + [("PeriodicBoundary", {}, (S(None), S(None), 0)), POINT], True),
+    "flat_x": ((1, 19, 30), faces(4, (1, 2)) + [POINT], True),
+    "flat_y": ((33, 1, 18), faces(3, (2, 0)) + [POINT], True),
+    "cube": ((17, 18, 19), faces(4) + [POINT], True),
+    "no_faces": ((9, 7, 5), [POINT], True),
+    "thin_faces": ((11, 10, 23), faces(1) + [POINT], True),
+    "one_side": ((14, 13, 12), [face(1, 1, 5), face(2, 0, 6), POINT], True),
+    "z_first": ((13, 12, 15), faces(3, (2, 0, 1)) + [POINT], True),
+    "mixed_order": ((13, 12, 15), [face(0, 0, 3), face(1, 1, 3), face(0, 1, 3), face(1, 0, 3), POINT], False),
+    "overlapping_slabs": ((7, 12, 11), [face(0, 0, 5), face(0, 1, 5), POINT], False),
+    "periodic": ((10, 11, 12), faces(3, (0, 1)) + [("PeriodicBoundary", {}, (S(None), S(None), 0)), POINT], False),
+    "slabs_meet": ((8, 12, 11), [face(0, 0, 4), face(0, 1, 4), POINT], True),
+    "objects": ((18, 17, 16), faces(3) + [
+        ("Object", dict(permittivity=2.5), (S(4, 9), S(3, 8), S(5, 12))),
+        ("AbsorbingObject", dict(permittivity=1.5, conductivity=2e4), (S(8, 13), S(6, 11), S(2, 9))),
+        ("AnisotropicObject", dict(permittivity=2.0), (S(11, 15), S(9, 14), S(10, 13))), POINT], True),
+    "five_points": ((15, 14, 13), faces(3) + [("PointSource", dict(period=7 + n), (3 + n, 4 + n, 5)) for n in range(5)]
+                    + [("PointSource", dict(period=8), (3, 4, 5))], True),
+    "lines": ((20, 17, 15), faces(3) + [
+        ("LineSource", dict(period=11), (4, S(3, 12), 7)),
+        ("LineSource", dict(period=12), (S(5, 15), S(2, 9), 9)),
+        ("LineSource", dict(period=13), ([9, 5, 12], [8, 8, 3], [4, 4, 10]))], True),
+    "repeated_cell": ((14, 13, 12), faces(3) + [
+        POINT, ("LineDetector", {}, ([4, 5, 4], [6, 6, 6], [7, 7, 7]))], False),
+    "plane": ((14, 19, 17), faces(3) + [
+        ("PlaneSource", dict(period=15, polarization="y"), (5, S(4, 15), S(3, 12))),
+        ("LineSource", dict(period=11), (5, S(3, 12), 7))], True),
+    "detectors": ((17, 15, 14), faces(3) + [
+        ("LineDetector", {}, (S(2, 14), 7, 6)), ("LineDetector", {}, (S(3, 13), S(2, 12), S(1, 11))),
+        ("BlockDetector", {}, (S(4, 7), S(9, 9), S(2, 11))), POINT], True),
+    "many_tiles": ((21, 34, 67), faces(6) + [POINT], True),
+}
+BACKENDS = ("hip.float64", "hip.float32", "hip.float32c")
+RUNS = (4, 1, 3)  # even, single and odd runs, half steps and an edit between them
+
+
+def build(fdtd, name, seed=0):
+    shape, comps, _ = FORMS[name]
+    rng = np.random.RandomState(seed)
+    eps = rng.uniform(1.0, 4.0, size=shape + (3,))
+    mu = rng.uniform(1.0, 2.0, size=shape + (3,))
+    grid = fdtd.Grid(shape, grid_spacing=100e-9, courant_number=0.5, permittivity=torch.from_numpy(eps),
+                     permeability=torch.from_numpy(mu))
+    for kind, params, key in comps:
+        if key == "mid":
+            key = tuple(n // 2 for n in shape)
+        grid[key] = getattr(fdtd, kind)(**params)
+    grid.E = torch.from_numpy(0.1 * rng.randn(*shape, 3))
+    grid.H = torch.from_numpy(0.1 * rng.randn(*shape, 3))
+    return grid
+
+
+def state(grid):
+    out = [grid._E_rec, grid._H_rec] if grid.compensated else [grid._E, grid._H]
+    for b in grid.boundaries:
+        out += [t for t in (getattr(b, "_psiE", None), getattr(b, "_psiH", None)) if t is not None]
+    for d in grid.detectors:
+        out += [d.trace("E"), d.trace("H")]
+    return [t.clone() for t in out]
+
+
+def advance(grid):
+    """RUNS with a state after each, half steps and a material edit between."""
+    out = []
+    for n in RUNS:
+        grid.run(n, progress_bar=False)
+        out += state(grid)
+        grid.update_E()
+        grid.update_H()
+        grid.time_steps_passed += 1
+        grid.inverse_permittivity[0] *= 0.5
+    return out
+
+
+def whole(grid):
+    """Whether the grid's plan took whole steps."""
+    return isinstance(grid._plan.step_buf, torch.Tensor)
+
+
+def differences(fdtd, name, backend):
+    """Names of what is wrong: differing states, or the other route taken."""
+    fdtd.set_backend(backend)
+    keep = os.environ.get("FDTD_HIP_STEP")
+    try:
+        os.environ["FDTD_HIP_STEP"] = "0"
+        half = build(fdtd, name)
+        want = advance(half)
+        os.environ["FDTD_HIP_STEP"] = "1"
+        grid = build(fdtd, name)
+        got = advance(grid)
+    finally:
+        if keep is None:
+            os.environ.pop("FDTD_HIP_STEP", None)
+        else:
+            os.environ["FDTD_HIP_STEP"] = keep
+    bad = [f"state {i}" for i, (a, b) in enumerate(zip(got, want))
+           if not torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))]
+    if whole(half):
+        bad.append("half steps were asked for")
+    if whole(grid) != FORMS[name][2]:
+        bad.append(f"whole steps: {whole(grid)}")
+    return bad
