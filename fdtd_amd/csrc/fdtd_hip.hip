@@ -104,6 +104,11 @@ struct FdtdPlan {
   // device tables
   void* dev = nullptr;
   FaceDev* d_faces = nullptr;  // faces in boundary registration order
+  Side* d_main_sides = nullptr;  // the fused faces by side (main_form)
+  int main_t[6] = {0, 0, 0, 0, 0, 0};
+  int main_order = -1;  // their order, or -1: the general form of the main kernels
+  uint32_t* d_obj_tiles = nullptr;  // object_tiles, or null: one launch
+  int64_t n_obj_tiles = 0;
   ObjDev* d_objs = nullptr;
   SrcDev* d_srcs = nullptr;
   DetDev* d_dets = nullptr;
@@ -159,6 +164,7 @@ struct FdtdBatch {
   int64_t total = 0;
   bool cyclic = false;        // x-chunks dealt cyclically to the XCDs (BatchArgs)
   bool objs = false;          // some grid has objects: the E kernel variant with them
+  bool any = false;           // some grid needs the general form of the kernels
   // captured steps
   hipStream_t gstream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
@@ -281,6 +287,35 @@ MatPalette<float> make_mat(const FdtdPlan* p, bool mu) {
   return {mu ? p->mu_id : p->eps_id, mu ? p->mu_tab : p->eps_tab};
 }
 
+// The order in which a cell's faces along the three axes are applied (two bits
+// an axis), the plan's first n faces, or -1 when no one order holds for every combination of
+// sides (the order is the faces' registration order), or when a side has
+// several faces or the two slabs of an axis overlap.
+int face_order(const FdtdPlan* p, size_t n_faces) {
+  int rank[3][2], t[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  for (size_t f = 0; f < n_faces; ++f) {
+    const FaceHost& fh = p->faces[f];
+    if (t[fh.axis][fh.high]) return -1;
+    t[fh.axis][fh.high] = fh.t;
+    rank[fh.axis][fh.high] = (int)f;
+  }
+  const int n[3] = {p->d.nx, p->d.ny, p->d.nz};
+  for (int ax = 0; ax < 3; ++ax)
+    if (t[ax][0] + t[ax][1] > n[ax]) return -1;
+  // whether every face along a comes before every face along b
+  auto before = [&](int a, int b) {
+    for (int u = 0; u < 2; ++u)
+      for (int v = 0; v < 2; ++v)
+        if (t[a][u] && t[b][v] && rank[a][u] > rank[b][v]) return false;
+    return true;
+  };
+  int ax[3] = {0, 1, 2};
+  do {
+    if (before(ax[0], ax[1]) && before(ax[0], ax[2]) && before(ax[1], ax[2])) return ax[0] | ax[1] << 2 | ax[2] << 4;
+  } while (std::next_permutation(ax, ax + 3));
+  return -1;
+}
+
 template <class FS, class MS>
 MainArgs<FS, MS> main_args(const FdtdPlan* p, bool is_H) {
   MainArgs<FS, MS> a{};
@@ -291,6 +326,9 @@ MainArgs<FS, MS> main_args(const FdtdPlan* p, bool is_H) {
   a.M = make_mat<MS>(p, is_H);
   a.faces = p->d_faces;
   a.nfaces = p->n_fused;
+  a.sides = p->d_main_sides;
+  for (int s = 0; s < 6; ++s) a.t[s] = p->main_t[s];
+  a.order = p->main_order;
   a.objs = p->d_objs;
   a.nobjs = is_H ? 0 : (int)p->objs.size();
   const int bzs = lanes_shift(p->d.nz);
@@ -301,6 +339,47 @@ MainArgs<FS, MS> main_args(const FdtdPlan* p, bool is_H) {
   a.flat = p->flat ? p->block_threads : 0;
   a.npts = 0;
   return a;
+}
+
+// Whether a's launch takes the main form of the kernels: faces that have an
+// order (face_order), and cells within 32-bit byte offsets of a chunk's first
+// plane. Others take the general form.
+template <class FS, class MS>
+bool main_form(const MainArgs<FS, MS>& a) {
+  return a.order >= 0 && ((uint64_t)a.cx + 2) * (uint64_t)a.d.px * std::max(FS::kCell, MS::kCell) < (uint64_t)1 << 32;
+}
+
+// Tiles of the main kernels that meet an object, in order, where an E half
+// step is split in two launches: the main form over the wavefronts that meet
+// none, the general form over these tiles. A second launch costs ~6 us, the
+// main form saves 10-14 % of the time of the general one (float32
+// 200x190x180 87 -> 80 us, 512x512x384 1045 -> 900): grids of 4M cells and more.
+std::vector<uint32_t> object_tiles(const FdtdPlan* p) {
+  std::vector<uint32_t> out;
+  const char* env = getenv("FDTD_HIP_OBJECT_TILES");  // 0: never, 1: any size
+  if (p->objs.empty() || p->dtype == FDTD_F32C || (env ? atoi(env) == 0 : grid_cells(p) < (int64_t)1 << 22)) return out;
+  const Dims& d = p->d;
+  const int bzs = lanes_shift(d.nz), bz = 1 << bzs, by = std::max(1, p->block_threads >> bzs);
+  const int flat = p->flat ? p->block_threads : 0;
+  const int64_t per = plane_tiles(d, bzs, by, flat), nch = (d.nx + p->cx - 1) / p->cx;
+  std::vector<char> has(per);
+  for (int64_t c = 0; c < nch; ++c) {
+    const int i0 = (int)c * p->cx, i1 = std::min(i0 + p->cx, d.nx);
+    std::fill(has.begin(), has.end(), 0);
+    for (const ObjHost& o : p->objs) {
+      if (o.x1 <= i0 || o.x0 >= i1) continue;
+      for (int j = o.y0; j < o.y1; ++j) {
+        // the tiles of the object's cells of row j
+        const int64_t first = flat ? ((int64_t)j * d.nz + o.z0) / flat : (int64_t)(j / by) * ((d.nz + bz - 1) / bz) + o.z0 / bz;
+        const int64_t last = flat ? ((int64_t)j * d.nz + o.z1 - 1) / flat
+                                  : (int64_t)(j / by) * ((d.nz + bz - 1) / bz) + (o.z1 - 1) / bz;
+        for (int64_t t = first; t <= last; ++t) has[t] = 1;
+      }
+    }
+    for (int64_t t = 0; t < per; ++t)
+      if (has[t]) out.push_back((uint32_t)(c * per + t));
+  }
+  return out;
 }
 
 // threads per workgroup of main-kernel arguments a
@@ -315,36 +394,56 @@ void launch_main(const FdtdPlan* p, const MainArgs<FS, MS>& a, bool is_H, hipStr
   const unsigned nchunks = (unsigned)((p->d.nx + a.cx - 1) / a.cx);
   // x-chunks dealt cyclically to the 8 XCDs (xcd_chunk_tile): whole rounds of 8
   const dim3 grid(tiles * (a.cyclic ? (nchunks + 7) / 8 * 8 : nchunks)), block(block_of(a));
-  if (a.rec) {  // recording forward pass of a gradient (plain storage)
-    if (a.nobjs)
-      hipLaunchKernelGGL((k_main_E<FS, MS, O, true, true, true>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((k_main_E<FS, MS, O, false, true, true>), grid, block, 0, st, a);
-  } else if (p->nontemporal) {
-    if (is_H)
+  const bool main = main_form(a);
+  if (is_H) {
+    if (!main)
+      hipLaunchKernelGGL((k_any_H<FS, MS>), grid, block, 0, st, a);
+    else if (p->nontemporal)
       hipLaunchKernelGGL((k_main_H<FS, MS, true>), grid, block, 0, st, a);
-    else if (a.nobjs)
-      hipLaunchKernelGGL((k_main_E<FS, MS, O, true, true, false>), grid, block, 0, st, a);
     else
-      hipLaunchKernelGGL((k_main_E<FS, MS, O, false, true, false>), grid, block, 0, st, a);
-  } else {
-    if (is_H)
       hipLaunchKernelGGL((k_main_H<FS, MS, false>), grid, block, 0, st, a);
-    else if (a.nobjs)
-      hipLaunchKernelGGL((k_main_E<FS, MS, O, true, false, false>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((k_main_E<FS, MS, O, false, false, false>), grid, block, 0, st, a);
+    return;
   }
+  if constexpr (FS::kRecords) {
+    // the records' decoding leaves no registers for the main form: 213 us
+    // against 205 for this one at 256^3
+    if (a.nobjs)
+      hipLaunchKernelGGL((k_any_E<FS, MS, O, true, false>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_any_E<FS, MS, O, false, false>), grid, block, 0, st, a);
+  } else if (a.rec) {  // recording forward pass of a gradient
+    hipLaunchKernelGGL((k_any_E<FS, MS, O, true, true>), grid, block, 0, st, a);
+  } else if (!main || (a.nobjs && !p->d_obj_tiles)) {
+    hipLaunchKernelGGL((k_any_E<FS, MS, O, true, false>), grid, block, 0, st, a);
+  } else if (a.nobjs) {
+    hipLaunchKernelGGL((k_main_E<FS, MS, true, true>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((k_object_E<FS, MS, O>), dim3((unsigned)p->n_obj_tiles), block, 0, st, a,
+                       (const uint32_t*)p->d_obj_tiles);
+  } else if (p->nontemporal) {
+    hipLaunchKernelGGL((k_main_E<FS, MS, false, true>), grid, block, 0, st, a);
+  } else {
+    hipLaunchKernelGGL((k_main_E<FS, MS, false, false>), grid, block, 0, st, a);
+  }
+}
+
+template <class FS, class MS>
+void fold_points(const FdtdPlan* p, MainArgs<FS, MS>& a) {
+  a.npts = (int32_t)p->srcs.size();
+  for (int s = 0; s < a.npts; ++s) {
+    const int64_t c = p->srcs[s].cells[0];
+    a.pt_cell[s] = c;
+    a.pt_plane[s] = (int32_t)(c / p->d.px);
+    a.pt_at[s] = (int32_t)(c % p->d.px);
+  }
+  a.wave = p->wave;
+  a.wave_cap = p->wave_cap;
 }
 
 template <class FS, class MS, typename O>
 int launch_half(FdtdPlan* p, bool is_H, int64_t q, hipStream_t st) {
   MainArgs<FS, MS> a = main_args<FS, MS>(p, is_H);
   if (!is_H && p->fold_points) {
-    a.npts = (int32_t)p->srcs.size();
-    for (int s = 0; s < a.npts; ++s) a.pt_cell[s] = p->srcs[s].cells[0];
-    a.wave = p->wave;
-    a.wave_cap = p->wave_cap;
+    fold_points(p, a);
     a.q = q;
   }
   if (!is_H && p->rec_curl) {
@@ -495,35 +594,6 @@ Box cells_box(const FdtdPlan* p, const std::vector<int64_t>& cells) {
   return b;
 }
 
-// The order in which a cell's faces along the three axes are applied, as
-// StepArgs::order, or -1 when no one order holds for every combination of
-// sides (the order is the faces' registration order), or when a side has
-// several faces or the two slabs of an axis overlap.
-int face_order(const FdtdPlan* p) {
-  int rank[3][2], t[3][2] = {{0, 0}, {0, 0}, {0, 0}};
-  for (size_t f = 0; f < p->faces.size(); ++f) {
-    const FaceHost& fh = p->faces[f];
-    if (t[fh.axis][fh.high]) return -1;
-    t[fh.axis][fh.high] = fh.t;
-    rank[fh.axis][fh.high] = (int)f;
-  }
-  const int n[3] = {p->d.nx, p->d.ny, p->d.nz};
-  for (int ax = 0; ax < 3; ++ax)
-    if (t[ax][0] + t[ax][1] > n[ax]) return -1;
-  // whether every face along a comes before every face along b
-  auto before = [&](int a, int b) {
-    for (int u = 0; u < 2; ++u)
-      for (int v = 0; v < 2; ++v)
-        if (t[a][u] && t[b][v] && rank[a][u] > rank[b][v]) return false;
-    return true;
-  };
-  int ax[3] = {0, 1, 2};
-  do {
-    if (before(ax[0], ax[1]) && before(ax[0], ax[2]) && before(ax[1], ax[2])) return ax[0] | ax[1] << 2 | ax[2] << 4;
-  } while (std::next_permutation(ax, ax + 3));
-  return -1;
-}
-
 // Whether the plan's whole step can run as one kernel: nothing but the E half
 // step's own update may stand between a cell's E and the H that reads it. A
 // periodic copy (of an axis longer than one cell) and a soft source, which
@@ -545,7 +615,7 @@ bool step_eligible(const FdtdPlan* p) {
   const int64_t most = (int64_t)1 << (flat ? 21 : (p->dtype == FDTD_F32 ? 17 : 20));
   const char* env = getenv("FDTD_HIP_STEP");
   if (env ? atoi(env) == 0 : grid_cells(p) > most) return false;
-  if (face_order(p) < 0 || p->srcs.size() > 32 || p->dets.size() > 32 || !p->curs.empty()) return false;
+  if (face_order(p, p->faces.size()) < 0 || p->srcs.size() > 32 || p->dets.size() > 32 || !p->curs.empty()) return false;
   if (p->d.cs >= (int64_t)1 << 28) return false;  // 32-bit byte offsets
   for (const Bnd& b : p->stages) {
     const int n = b.index == 0 ? p->d.nx : (b.index == 1 ? p->d.ny : p->d.nz);
@@ -677,7 +747,7 @@ int build_step_tables(FdtdPlan* p) {
     std::memcpy(host.data() + o_d + i * sizeof(sd), &sd, sizeof(sd));
   }
   step_shape(p, p->step_tile);
-  p->step_order = face_order(p);
+  p->step_order = face_order(p, p->faces.size());
   FDTD_HIP(hipMemcpy(p->step_dev, host.data(), total, hipMemcpyHostToDevice));
   for (int h = 0; h < 2; ++h) p->d_sides[h] = reinterpret_cast<StepSide*>(base + o_f[h]);
   p->d_back = reinterpret_cast<CopySeg*>(base + o_b);
@@ -986,14 +1056,14 @@ bool batch_cyclic(const std::vector<FdtdPlan*>& plans) {
 template <class FS, class MS>
 void batch_tables(const std::vector<FdtdPlan*>& plans, int block_threads, int cx, bool cyclic,
                   std::vector<MainArgs<FS, MS>>& sE, std::vector<MainArgs<FS, MS>>& sH, std::vector<int64_t>& first,
-                  std::vector<int32_t>& rot, bool& objs) {
+                  std::vector<int32_t>& rot, bool& objs, bool& any) {
   using MA = MainArgs<FS, MS>;
   const size_t n = plans.size();
   sE.assign(n, MA{});
   sH.assign(n, MA{});
   first.assign(n + 1, 0);
   rot.assign(n, 0);
-  objs = false;
+  objs = any = false;
   int64_t chunks = 0;  // chunks of the grids before this one
   for (size_t i = 0; i < n; ++i) {
     FdtdPlan* p = plans[i];
@@ -1005,12 +1075,10 @@ void batch_tables(const std::vector<FdtdPlan*>& plans, int block_threads, int cx
       a->flat = p->flat ? block_threads : 0;
     }
     if (p->fold_points) {
-      aE.npts = (int32_t)p->srcs.size();
-      for (int s = 0; s < aE.npts; ++s) aE.pt_cell[s] = p->srcs[s].cells[0];
-      aE.wave = p->wave;
-      aE.wave_cap = p->wave_cap;
+      fold_points(p, aE);
     }
     objs = objs || aE.nobjs > 0;
+    any = any || !main_form(aE) || !main_form(aH);
     sE[i] = aE;
     sH[i] = aH;
     const int64_t per = plane_tiles(p->d, aE.bz_shift, aE.by, aE.flat), nch = (p->d.nx + aE.cx - 1) / aE.cx;
@@ -1030,6 +1098,7 @@ struct BatchImage {
   int64_t total = 0;  // positions of the work list
   bool cyclic = false;
   bool objs = false;
+  bool any = false;
 };
 
 int batch_image(const std::vector<FdtdPlan*>& plans, int block_threads, int cx, BatchImage& img) {
@@ -1040,7 +1109,7 @@ int batch_image(const std::vector<FdtdPlan*>& plans, int block_threads, int cx, 
     std::vector<int64_t> first;
     std::vector<int32_t> rot;
     img.cyclic = batch_cyclic(plans);
-    batch_tables<FS, MS>(plans, block_threads, cx, img.cyclic, sE, sH, first, rot, img.objs);
+    batch_tables<FS, MS>(plans, block_threads, cx, img.cyclic, sE, sH, first, rot, img.objs, img.any);
     img.total = first[n];
     if (img.total >= (int64_t)1 << 31) return fail(-1, "batch has too many work items");
     img.oE = 0;
@@ -1077,6 +1146,7 @@ int batch_upload(FdtdBatch* b) {
   b->total = img.total;
   b->cyclic = img.cyclic;
   b->objs = img.objs;
+  b->any = img.any;
   FDTD_HIP(hipMalloc(&b->dev, img.bytes.size()));
   FDTD_HIP(hipMemcpy(b->dev, img.bytes.data(), img.bytes.size(), hipMemcpyHostToDevice));
   char* base = reinterpret_cast<char*>(b->dev);
@@ -1104,6 +1174,7 @@ struct BatchTables {
   int64_t total;
   int64_t* q;
   bool cyclic;
+  bool any;  // some grid needs the general form of the kernels
 };
 
 // nsteps batched steps on stream st (the time index already set on the
@@ -1118,18 +1189,24 @@ int batch_launch_tables(const FdtdPlan* p0, const BatchTables& t, bool objs, int
     aH.sims = reinterpret_cast<const MainArgs<FS, MS>*>(t.sims_H);
     const bool loop = groups < t.total;  // a persistent grid of workgroups
     for (int64_t s = 0; s < nsteps; ++s) {
-      if (objs && loop)
-        hipLaunchKernelGGL((k_batch_E<FS, MS, O, true, true, true>), grid, block, 0, st, aE);
-      else if (objs)
-        hipLaunchKernelGGL((k_batch_E<FS, MS, O, true, true, false>), grid, block, 0, st, aE);
+      if (t.any || objs) {  // objects, or a grid that takes the general form: all do
+        if (loop)
+          hipLaunchKernelGGL((k_batch_E<FS, MS, O, true, true, kObjects>), grid, block, 0, st, aE);
+        else
+          hipLaunchKernelGGL((k_batch_E<FS, MS, O, true, false, kObjects>), grid, block, 0, st, aE);
+      } else {
+        constexpr int form = FS::kRecords ? kGeneral : kMainForm;
+        if (loop)
+          hipLaunchKernelGGL((k_batch_E<FS, MS, O, true, true, form>), grid, block, 0, st, aE);
+        else
+          hipLaunchKernelGGL((k_batch_E<FS, MS, O, true, false, form>), grid, block, 0, st, aE);
+      }
+      if (t.any)
+        hipLaunchKernelGGL((k_batch_H<FS, MS, true, true, true>), grid, block, 0, st, aH);
       else if (loop)
-        hipLaunchKernelGGL((k_batch_E<FS, MS, O, false, true, true>), grid, block, 0, st, aE);
+        hipLaunchKernelGGL((k_batch_H<FS, MS, true, true, false>), grid, block, 0, st, aH);
       else
-        hipLaunchKernelGGL((k_batch_E<FS, MS, O, false, true, false>), grid, block, 0, st, aE);
-      if (loop)
-        hipLaunchKernelGGL((k_batch_H<FS, MS, true, true>), grid, block, 0, st, aH);
-      else
-        hipLaunchKernelGGL((k_batch_H<FS, MS, true, false>), grid, block, 0, st, aH);
+        hipLaunchKernelGGL((k_batch_H<FS, MS, true, false, false>), grid, block, 0, st, aH);
     }
     FDTD_HIP(hipGetLastError());
     return 0;
@@ -1137,7 +1214,7 @@ int batch_launch_tables(const FdtdPlan* p0, const BatchTables& t, bool objs, int
 }
 
 int batch_launch(FdtdBatch* b, int64_t nsteps, hipStream_t st) {
-  const BatchTables t{b->sims_E, b->sims_H, b->first, b->item_sim, b->rot, b->total, b->q, b->cyclic};
+  const BatchTables t{b->sims_E, b->sims_H, b->first, b->item_sim, b->rot, b->total, b->q, b->cyclic, b->any};
   return batch_launch_tables(b->plans[0], t, b->objs, batch_groups(b), b->block_threads, nsteps, st);
 }
 
@@ -1151,7 +1228,8 @@ BatchTables image_tables(const BatchImage& img, void* base) {
                      reinterpret_cast<const int32_t*>(c + img.oR),
                      img.total,
                      reinterpret_cast<int64_t*>(c + img.oQ),
-                     img.cyclic};
+                     img.cyclic,
+                     img.any};
 }
 
 // ----------------------------------------------- batch without allocation
@@ -1507,6 +1585,8 @@ int fdtd_plan_finalize(FdtdPlan* p) {
   size_t off = 0;
   const size_t o_faces = off;
   off = align_up(off + nf * sizeof(FaceDev));
+  const size_t o_sides = off;
+  off = align_up(off + 6 * sizeof(Side));
   const size_t o_objs = off;
   off = align_up(off + no * sizeof(ObjDev));
   const size_t o_srcs = off;
@@ -1535,8 +1615,12 @@ int fdtd_plan_finalize(FdtdPlan* p) {
     o_dcell[i] = off;
     off = align_up(off + p->dets[i].cells.size() * sizeof(int64_t));
   }
+  const std::vector<uint32_t> obj_tiles = object_tiles(p);
+  const size_t o_otiles = off;
+  off = align_up(off + obj_tiles.size() * sizeof(uint32_t));
   const size_t total = off > 0 ? off : 256;
   std::vector<unsigned char> host(total, 0);
+  if (!obj_tiles.empty()) std::memcpy(host.data() + o_otiles, obj_tiles.data(), obj_tiles.size() * sizeof(uint32_t));
   char* base = nullptr;
   FDTD_HIP(hipMalloc(&p->dev, total));
   base = reinterpret_cast<char*>(p->dev);
@@ -1561,6 +1645,22 @@ int fdtd_plan_finalize(FdtdPlan* p) {
     fd.psiH = f.psiH;
     fd.slab = plane_cells(p, f.axis) * f.t;
     p->h_faces.push_back(fd);
+  }
+  // the fused faces by side, if they have one order for every cell
+  p->main_order = face_order(p, (size_t)p->n_fused);
+  if (const char* env = getenv("FDTD_HIP_GENERAL"))  // the general form, to check that both agree
+    if (atoi(env) != 0) p->main_order = -1;
+  std::fill(p->main_t, p->main_t + 6, 0);
+  for (int i = 0; i < p->n_fused; ++i) {
+    const FaceDev& fd = p->h_faces[i];
+    const size_t comp = (size_t)fd.slab * value_bytes(p);
+    if (comp >= (size_t)1 << 32) p->main_order = -1;  // 32-bit byte offsets into a component
+    if (p->main_order < 0) break;
+    char *psiE = static_cast<char*>(fd.psiE), *psiH = static_cast<char*>(fd.psiH);
+    const Side sd{{psiE, psiE + comp}, {psiH, psiH + comp}, fd.bE, fd.cE, fd.bH, fd.cH};
+    const int s = fd.axis * 2 + (fd.high ? 1 : 0);
+    std::memcpy(host.data() + o_sides + s * sizeof(Side), &sd, sizeof(Side));
+    p->main_t[s] = fd.t;
   }
   // fused faces first (registration order), then the staged ones
   std::vector<FaceDev> ordered;
@@ -1619,6 +1719,9 @@ int fdtd_plan_finalize(FdtdPlan* p) {
   }
   FDTD_HIP(hipMemcpy(p->dev, host.data(), total, hipMemcpyHostToDevice));
   p->d_faces = reinterpret_cast<FaceDev*>(base + o_faces);
+  p->d_main_sides = reinterpret_cast<Side*>(base + o_sides);
+  p->n_obj_tiles = (int64_t)obj_tiles.size();
+  p->d_obj_tiles = obj_tiles.empty() ? nullptr : reinterpret_cast<uint32_t*>(base + o_otiles);
   p->d_objs = reinterpret_cast<ObjDev*>(base + o_objs);
   p->d_srcs = reinterpret_cast<SrcDev*>(base + o_srcs);
   p->d_dets = reinterpret_cast<DetDev*>(base + o_dets);

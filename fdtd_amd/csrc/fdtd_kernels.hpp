@@ -127,6 +127,43 @@ __device__ __forceinline__ gptr<T> gp(T* p) {
   return (gptr<T>)p;
 }
 
+// Read-only tables: the constant address space, so that uniform reads are
+// scalar loads whatever the kernel stores in between.
+template <typename T>
+using cptr = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ cptr<T> cp(const T* p) {
+  return (cptr<T>)p;
+}
+
+// Keeps a work-item's offset out of loop-invariant address arithmetic: the
+// compiler would otherwise add it to each array's base outside the loop (a
+// 64-bit register pair per array and component, and a 64-bit addition per
+// access) instead of using the scalar base + 32-bit offset form of an access.
+__device__ __forceinline__ void opaque(uint32_t& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(x));
+#endif
+}
+// The same for a table's address: what is read through it is read again each
+// time round a loop rather than kept in scalar registers across it.
+template <typename P>
+__device__ __forceinline__ void opaque_table(P& p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(p));
+#endif
+}
+
+// Whether any lane of the wavefront has x (a host build runs its work-items
+// one by one: the work-item's own x).
+__device__ __forceinline__ bool wave_any(bool x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_ballot_w64(x) != 0;
+#else
+  return x;
+#endif
+}
+
 // p[0] of an array whose base is the same for the whole wavefront, `off` bytes
 // further on.
 template <typename T>
@@ -428,7 +465,9 @@ struct MatArray {
 #pragma unroll
     for (int c = 0; c < 3; ++c) m[c] = (R)ld_stream<NT>(p + c * cs + i);
   }
-  // as PlainField's: what is loaded for a cell, and its three values
+  // as PlainField's: what is loaded for a cell, and its three values (kAhead:
+  // what is loaded leads to them, and the marching kernels load it a plane ahead)
+  static constexpr bool kAhead = false;
   static constexpr uint32_t kCell = sizeof(S);
   struct Own {
     S v[3];
@@ -456,6 +495,7 @@ struct MatPalette {
 #pragma unroll
     for (int c = 0; c < 3; ++c) m[c] = (R)gp(tab)[3 * k + c];
   }
+  static constexpr bool kAhead = true;
   static constexpr uint32_t kCell = 1;
   using Own = uint8_t;
   template <bool NT>
@@ -540,6 +580,166 @@ __device__ __forceinline__ void pml_cell(const FaceDev* __restrict__ faces, int 
                    v[2]);
 }
 
+// The face of one side of the grid as the main kernels read it: its two psi
+// components and its profiles (a table of 6, [axis][low/high]).
+struct Side {
+  void* psiE[2];
+  void* psiH[2];
+  const double* bE;
+  const double* cE;
+  const double* bH;
+  const double* cH;
+};
+
+// Two psi values of one cell and face, `off` bytes into their arrays.
+template <typename T>
+struct Psi {
+  T p0, p1;
+  __device__ __forceinline__ void load(const void* a0, const void* a1, uint32_t off) {
+    p0 = ld_stream<false>(split_ptr(reinterpret_cast<const T*>(a0), off));
+    p1 = ld_stream<false>(split_ptr(reinterpret_cast<const T*>(a1), off));
+  }
+  __device__ __forceinline__ void store(void* a0, void* a1, uint32_t off) const {
+    st_stream<false>(split_ptr(reinterpret_cast<T*>(a0), off), p0);
+    st_stream<false>(split_ptr(reinterpret_cast<T*>(a1), off), p1);
+  }
+  // psi <- psi b, plus (difference) c where the slab has both of its cells
+  __device__ __forceinline__ void advance(T b, T c, bool inner, T d0, T d1) {
+    p0 = p0 * b;
+    p1 = p1 * b;
+    if (inner) {
+      p0 = p0 + d0 * c;
+      p1 = p1 + d1 * c;
+    }
+  }
+};
+
+// The CPML of one cell column of a tile, for plans with at most one face a side
+// whose slabs do not overlap (a cell is then in one slab per axis at most).
+// Which slabs of the y and z axes the column is in and its place there do not
+// change from plane to plane and are found once; every psi value and
+// coefficient of a plane is loaded with the plane's fields, before any of them
+// is waited for; and a wavefront that meets no slab does nothing for them.
+template <bool IS_E, typename T>
+struct TilePml {
+  enum : uint32_t { kLoY = 1, kHiY = 2, kLoZ = 4, kHiZ = 8, kInY = 16, kInZ = 32 };
+  cptr<Side> sides;
+  uint32_t flags = 0;  // the column's slabs; kIn*: the slab has both cells of the difference
+  uint32_t qy = 0, qz = 0, ystep = 0, zstep = 0;  // byte offsets in the psi arrays, and a plane further
+  uint32_t ly = 0, lz = 0;  // byte offsets in the profiles
+  bool any_y, any_z;  // some column of the wavefront is in a y (z) slab
+  double by, cy, bz, cz;
+  Psi<T> px, py, pz;
+  int xs, xl;  // the plane's x slab (side, index), -1: none
+  uint32_t qx;
+
+  template <class A>
+  __device__ __forceinline__ void init(const A& a, int i, int j, int k) {
+    const Dims& d = a.d;
+    sides = cp(a.sides);
+    const auto inner = [](int l, int t) { return IS_E ? l >= 1 : l <= t - 2; };
+    if (j < a.t[2] || j >= d.ny - a.t[3]) {
+      const bool lo = j < a.t[2];
+      const int t = lo ? a.t[2] : a.t[3], l = lo ? j : j - (d.ny - t);
+      ystep = (uint32_t)(t * d.nz) * (uint32_t)sizeof(T);
+      qy = (uint32_t)i * ystep + (uint32_t)(l * d.nz + k) * (uint32_t)sizeof(T);
+      flags |= (lo ? kLoY : kHiY) | (inner(l, t) ? kInY : 0);
+      ly = (uint32_t)l * (uint32_t)sizeof(double);
+    }
+    if (k < a.t[4] || k >= d.nz - a.t[5]) {
+      const bool lo = k < a.t[4];
+      const int t = lo ? a.t[4] : a.t[5], l = lo ? k : k - (d.nz - t);
+      zstep = (uint32_t)(t * d.ny) * (uint32_t)sizeof(T);
+      qz = (uint32_t)i * zstep + (uint32_t)(j * t + l) * (uint32_t)sizeof(T);
+      flags |= (lo ? kLoZ : kHiZ) | (inner(l, t) ? kInZ : 0);
+      lz = (uint32_t)l * (uint32_t)sizeof(double);
+    }
+    any_y = wave_any(flags & (kLoY | kHiY));
+    any_z = wave_any(flags & (kLoZ | kHiZ));
+  }
+  __device__ __forceinline__ void fetch(int s, uint32_t& q, Psi<T>& p) const {
+    opaque(q);
+    const cptr<Side> sd = sides + s;
+    if (IS_E) p.load(sd->psiE[0], sd->psiE[1], q);
+    else p.load(sd->psiH[0], sd->psiH[1], q);
+  }
+  __device__ __forceinline__ void fetch(int s, uint32_t& q, uint32_t& l, Psi<T>& p, double& b, double& c) const {
+    fetch(s, q, p);
+    opaque(l);
+    const cptr<Side> sd = sides + s;
+    b = ld_stream<false>(split_ptr(IS_E ? sd->bE : sd->bH, l));
+    c = ld_stream<false>(split_ptr(IS_E ? sd->cE : sd->cH, l));
+  }
+  __device__ __forceinline__ void keep(int s, uint32_t& q, const Psi<T>& p) const {
+    opaque(q);
+    const cptr<Side> sd = sides + s;
+    if (IS_E) p.store(sd->psiE[0], sd->psiE[1], q);
+    else p.store(sd->psiH[0], sd->psiH[1], q);
+  }
+  // psi of plane i
+  template <class A>
+  __device__ __forceinline__ void load(const A& a, int i, uint32_t pc) {
+    opaque(flags);
+    opaque_table(sides);
+    xs = i < a.t[0] ? 0 : (i >= a.d.nx - a.t[1] ? 1 : -1);
+    if (xs >= 0) {
+      xl = xs ? i - (a.d.nx - a.t[1]) : i;
+      qx = ((uint32_t)xl * (uint32_t)(a.d.ny * a.d.nz) + pc) * (uint32_t)sizeof(T);
+      fetch(xs, qx, px);
+    }
+    if (any_y) {
+      if (flags & kLoY) fetch(2, qy, ly, py, by, cy);
+      if (flags & kHiY) fetch(3, qy, ly, py, by, cy);
+    }
+    if (any_z) {
+      if (flags & kLoZ) fetch(4, qz, lz, pz, bz, cz);
+      if (flags & kHiZ) fetch(5, qz, lz, pz, bz, cz);
+    }
+  }
+  // to the next plane of an E (up) or H (down) march
+  __device__ __forceinline__ void next_plane() {
+    qy = IS_E ? qy + ystep : qy - ystep;
+    qz = IS_E ? qz + zstep : qz - zstep;
+  }
+  // One step of the recursions and their terms in v (pml_face, above), the
+  // faces of a cell in the plan's order.
+  template <class A>
+  __device__ __forceinline__ void apply(const A& a, T zx, T yx, T zy, T xy, T yz, T xz, const T kc[3], T v[3]) {
+    if (!any_y && !any_z && xs < 0) return;
+#pragma nounroll
+    for (int n = 0; n < 3; ++n) {
+      const int ax = (a.order >> (2 * n)) & 3;
+      if (ax == 0 && xs >= 0) {
+        const cptr<Side> sd = sides + xs;
+        const T b = (T)cp(IS_E ? sd->bE : sd->bH)[xl], c = (T)cp(IS_E ? sd->cE : sd->cH)[xl];
+        px.advance(b, c, IS_E ? xl >= 1 : xl <= a.t[xs] - 2, zx, yx);
+        keep(xs, qx, px);
+        const T r0 = kc[1] * px.p0, r1 = kc[2] * px.p1;
+        v[1] = IS_E ? v[1] - r0 : v[1] + r0;
+        v[2] = IS_E ? v[2] + r1 : v[2] - r1;
+      } else if (ax == 1 && any_y) {
+        if (flags & (kLoY | kHiY)) {
+          py.advance((T)by, (T)cy, flags & kInY, zy, xy);
+          if (flags & kLoY) keep(2, qy, py);
+          if (flags & kHiY) keep(3, qy, py);
+          const T r0 = kc[0] * py.p0, r1 = kc[2] * py.p1;
+          v[0] = IS_E ? v[0] + r0 : v[0] - r0;
+          v[2] = IS_E ? v[2] - r1 : v[2] + r1;
+        }
+      } else if (ax == 2 && any_z) {
+        if (flags & (kLoZ | kHiZ)) {
+          pz.advance((T)bz, (T)cz, flags & kInZ, yz, xz);
+          if (flags & kLoZ) keep(4, qz, pz);
+          if (flags & kHiZ) keep(5, qz, pz);
+          const T r0 = kc[0] * pz.p0, r1 = kc[1] * pz.p1;
+          v[0] = IS_E ? v[0] - r0 : v[0] + r0;
+          v[1] = IS_E ? v[1] + r1 : v[1] - r1;
+        }
+      }
+    }
+  }
+};
+
 // E factor (1 - f) / (1 + f) of an absorbing object (objects.py:215). With
 // complex fields the reference divides in the dtype of f: complex (numpy's
 // division) when the object's permittivity is complex, real when it is real
@@ -609,6 +809,17 @@ __device__ __forceinline__ void objects_update_E(const ObjDev* __restrict__ objs
   }
 }
 
+// Whether a column (j, k) of the wavefront has, in x plane i, a cell inside an
+// object.
+__device__ __forceinline__ bool meets_objects(const ObjDev* objs, int nobjs, int i, int j, int k) {
+  for (int o = 0; o < nobjs; ++o) {
+    const cptr<ObjDev> ob = cp(objs) + o;
+    if (i < ob->x0 || i >= ob->x1) continue;
+    if (wave_any(j >= ob->y0 && j < ob->y1 && k >= ob->z0 && k < ob->z1)) return true;
+  }
+  return false;
+}
+
 // Logical tile of hardware workgroup w: workgroups are dealt round-robin to
 // the 8 XCDs (each with its own L2), so consecutive logical tiles -- which
 // share halo planes -- are given to the same XCD.
@@ -669,6 +880,11 @@ struct MainArgs {
   MS M;  // inv_eps or inv_mu
   const FaceDev* faces;
   int32_t nfaces;
+  // at most one face a side: the sides, their thicknesses (0: no face), and
+  // the order of a cell's faces (axes, two bits each)
+  const Side* sides;
+  int32_t t[6];
+  int32_t order;
   const ObjDev* objs;
   int32_t nobjs;
   int32_t bz_shift;  // block extent along z is 1 << bz_shift
@@ -681,6 +897,7 @@ struct MainArgs {
   // their cells, in registration order, and the waveform table
   int32_t npts;
   int64_t pt_cell[FOLDED_POINTS];
+  int32_t pt_plane[FOLDED_POINTS], pt_at[FOLDED_POINTS];  // x plane and place in it
   const double* wave;  // row s = source s
   int64_t wave_cap;
   int64_t q;
@@ -730,16 +947,19 @@ __device__ __forceinline__ void tile_column(const A& a, unsigned tile, int& j, i
   i1 = min(i0 + a.cx, d.nx);
 }
 
-// Main E kernel. A workgroup owns a (y, z) tile (tile_column) and marches
+// Main E kernel, general form: any faces (several a side, overlapping slabs,
+// an order that differs between sides: the face table is walked per cell) and
+// planes past the 32-bit offsets of the form below. A workgroup owns a (y, z) tile (tile_column) and marches
 // along x over a chunk of `cx` planes: the x-neighbours come from registers
 // of the previous plane, the y- and z-neighbours from cache (the rows were
 // just streamed in by this or the neighbouring wavefront). Every load of a
 // plane is issued unconditionally and at once, so a plane costs one memory
 // round trip: threads past the grid's edge read the nearest cell and store
 // nothing, and at the low edges the neighbour offset is 0 (the difference is
-// dropped).
-template <class FS, class MS, typename O, bool OBJS, bool NT, bool REC = false>
-__device__ __forceinline__ void main_E_tile(const MainArgs<FS, MS>& __restrict__ a, unsigned tile, int64_t q) {
+// dropped). ONLY: the wavefronts and planes that meet an object, which the
+// main form leaves (below).
+template <class FS, class MS, typename O, bool OBJS, bool NT, bool REC = false, bool ONLY = false>
+__device__ __forceinline__ void any_E_tile(const MainArgs<FS, MS>& __restrict__ a, unsigned tile, int64_t q) {
   using T = typename FS::R;
   const Dims d = a.d;
   int j, k, i0, i1;
@@ -760,7 +980,24 @@ __device__ __forceinline__ void main_E_tile(const MainArgs<FS, MS>& __restrict__
     }
   }
   typename MS::Key key = a.M.template key<NT>(cell);
+  bool skipped = false;
   for (int i = i0; i < i1; ++i, cell += sx) {
+    if constexpr (ONLY) {
+      if (!meets_objects(a.objs, a.nobjs, i, j, k)) {
+        skipped = true;
+        continue;
+      }
+      if (skipped) {  // nothing was carried from the plane before
+        skipped = false;
+        if constexpr (FS::kRecords) {
+          hrec = a.G.rec3(cell - sx);
+        } else {
+          hz_prev = a.G.template get_c<2>(cell - sx);
+          hy_prev = a.G.template get_c<1>(cell - sx);
+        }
+        key = a.M.template key<NT>(cell);
+      }
+    }
     T hv[3], m[3], e[3];
     const typename MS::Key kc_ = key;
     if (i + 1 < i1) key = a.M.template key<NT>(cell + sx);  // the next plane's, loaded with this one
@@ -822,6 +1059,98 @@ __device__ __forceinline__ void main_E_tile(const MainArgs<FS, MS>& __restrict__
   }
 }
 
+// Main E kernel: the form nearly every plan takes. As the general form, with
+// CPML per axis (TilePml: psi and coefficients loaded with the plane's fields)
+// and every access a scalar base plus a 32-bit offset that steps by a plane,
+// where the general form walks the face table cell by cell, each face a chain
+// of table, psi and coefficient loads, and forms 64-bit addresses. In float32
+// the kernels are bound by issue and by those chains rather than by bandwidth:
+// general -> main form 128^3 30.1 -> 24.7 us a launch, 24 grids of 64-160 cells
+// edge 0.887 -> 0.775 ms/step, 256^3 0.317 -> 0.293 ms/step; float64 at 256^3 is at
+// the fabric's rate either way (0.633 -> 0.626).
+// Nothing is guarded against work-items past the plane's edge: a wavefront of
+// them ends at once, and the ones beside the plane's last cell do that cell's
+// work, in lockstep with its own work-item, and store the same values (a
+// guarded block leaves loads unconsumed when it is skipped, and the wait for
+// them then stands between a plane's first loads and its others).
+// OBJS: wavefronts that meet an object in a plane leave it to k_object_E
+// (objects in this kernel would cost every cell the registers of their 3x3
+// products: spilling, it took 1.6x the general form's time in float64).
+template <class FS, class MS, bool OBJS, bool NT>
+__device__ __forceinline__ void main_E_tile(const MainArgs<FS, MS>& __restrict__ a, unsigned tile, int64_t q) {
+  using T = typename FS::R;
+  const Dims d = a.d;
+  int j, k, i0, i1;
+  bool act;
+  tile_column(a, tile, j, k, i0, i1, act);
+  if (!wave_any(act)) return;
+  const int ib = max(i0 - 1, 0);  // the offsets count from here
+  const int64_t base = (int64_t)ib * d.px;
+  const uint32_t pc = (uint32_t)(j * d.nz + k), at = (uint32_t)(i0 - ib) * (uint32_t)d.px + pc;
+  const uint32_t fstep = (uint32_t)d.px * FS::kCell, mstep = (uint32_t)d.px * MS::kCell;
+  uint32_t fo = at * FS::kCell, mo = at * MS::kCell;
+  const uint32_t dk = k > 0 ? FS::kCell : 0, dj = j > 0 ? (uint32_t)d.nz * FS::kCell : 0;
+  TilePml<true, T> pml;
+  pml.init(a, i0, j, k);
+  const T zero = T(0);
+  typename FS::Own hprev;  // H of plane i-1
+  typename MS::Own ahead{};
+  constexpr bool kAhead = MS::kAhead && !OBJS;
+  if constexpr (kAhead) ahead = a.M.template own<NT>(base, mo);
+  bool carried = false;  // hprev is plane i-1's
+  for (int i = i0; i < i1; ++i, fo += fstep, mo += mstep, pml.next_plane()) {
+    if constexpr (OBJS) {
+      if (meets_objects(a.objs, a.nobjs, i, j, k)) {
+        carried = false;
+        continue;
+      }
+    }
+    opaque(fo);
+    if constexpr (MS::kCell == FS::kCell) mo = fo;
+    // every load of the plane at once (the first plane's hprev among them:
+    // loaded ahead of the loop, it would be waited for before the others)
+    if (!carried) hprev = a.G.template own<false>(base, i > 0 ? fo - fstep : fo);
+    carried = true;
+    const typename FS::Own hown = a.G.template own<false>(base, fo);
+    const typename FS::Duo hk = a.G.template duo<0, 1>(base, fo - dk), hj = a.G.template duo<0, 2>(base, fo - dj);
+    typename MS::Own mat;
+    if constexpr (kAhead) {
+      mat = ahead;
+      if (i + 1 < i1) ahead = a.M.template own<NT>(base, mo + mstep);
+    } else {
+      mat = a.M.template own<NT>(base, mo);
+    }
+    const typename FS::Own eown = a.F.template own<NT>(base, fo);
+    pml.load(a, i, pc);
+    const T h0 = FS::template value<0>(hown), h1 = FS::template value<1>(hown), h2 = FS::template value<2>(hown);
+    // backward differences; an absent one contributes nothing (grid.py:67-74)
+    Diffs<T> df;
+    df.zy = dj ? h2 - FS::template value<0, 2, 2>(hj) : zero;
+    df.yz = dk ? h1 - FS::template value<0, 1, 1>(hk) : zero;
+    df.xz = dk ? h0 - FS::template value<0, 1, 0>(hk) : zero;
+    df.zx = i > 0 ? h2 - FS::template value<2>(hprev) : zero;
+    df.yx = i > 0 ? h1 - FS::template value<1>(hprev) : zero;
+    df.xy = dj ? h0 - FS::template value<0, 2, 0>(hj) : zero;
+    hprev = hown;
+    T e[3] = {FS::template value<0>(eown), FS::template value<1>(eown), FS::template value<2>(eown)};
+    T m[3], curl[3], kc[3];
+    a.M.values(mat, m);
+    curl[0] = (zero + df.zy) - df.yz;
+    curl[1] = (zero + df.xz) - df.zx;
+    curl[2] = (zero + df.yx) - df.xy;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      kc[c] = a.sc * m[c];
+      e[c] = e[c] + kc[c] * curl[c];
+    }
+    pml.apply(a, df.zx, df.yx, df.zy, df.xy, df.yz, df.xz, kc, e);
+    for (int s = 0; s < a.npts; ++s)  // sources.py:109, registration order
+      if (a.pt_plane[s] == i && (uint32_t)a.pt_at[s] == pc) e[2] = e[2] + (T)gp(a.wave)[s * a.wave_cap + q];
+    opaque(fo);
+    a.F.template put_own<NT>(base, fo, e);
+  }
+}
+
 // tiles per x-chunk and the number of x-chunks of a single-grid launch
 template <class FS, class MS>
 __device__ __forceinline__ void chunk_counts(const MainArgs<FS, MS>& a, unsigned& per_chunk, unsigned& nchunks) {
@@ -837,33 +1166,49 @@ __device__ __forceinline__ int64_t launch_tile(const MainArgs<FS, MS>& a, unsign
   return a.cyclic ? xcd_chunk_tile(blockIdx.x, per, nch) : (int64_t)xcd_tile(blockIdx.x, gridDim.x);
 }
 
-// Occupancy floor of the E kernels: the object variants otherwise take ~118
+// Occupancy floor of the E kernels: the general form otherwise takes ~118
 // VGPRs (4 waves per SIMD) for the anisotropic 3x3 path. Under a floor of 6
 // the double-precision ones fit in ~76 VGPRs without spilling, the float32
 // ones under a floor of 8 in ~46 (a floor of 8 makes the double ones spill);
 // complex128 values need twice the registers and keep a floor of 4. The
 // compensated kernels without objects fit 8 waves in 62 VGPRs (66 and 7
-// waves unbounded; 0.6 % faster per step at 256^3).
+// waves unbounded; 0.6 % faster per step at 256^3). The main forms fit under
+// the same floors.
 template <class FS, bool OBJS = true>
 struct EWaves {
-  static constexpr int value =
-      FS::kRecords && !OBJS ? 8 : (sizeof(typename FS::R) == 4 ? 8 : (sizeof(typename FS::R) == 8 ? 6 : 4));
+  static constexpr int bytes = sizeof(typename FS::R);
+  static constexpr int value = FS::kRecords && !OBJS ? 8 : (bytes == 4 ? 8 : (bytes == 8 ? 6 : 4));
 };
 
-template <class FS, class MS, typename O, bool OBJS, bool NT, bool REC>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(EWaves<FS, OBJS>::value)))
+template <class FS, class MS, bool OBJS, bool NT>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(EWaves<FS>::value)))
 k_main_E(MainArgs<FS, MS> a) {
   unsigned n;
   const int64_t t = launch_tile(a, n);
-  if (t >= 0) main_E_tile<FS, MS, O, OBJS, NT, REC>(a, (unsigned)t, a.q);
+  if (t >= 0) main_E_tile<FS, MS, OBJS, NT>(a, (unsigned)t, a.q);
 }
 
-// Main H kernel: the mirror image of the E kernel. Its differences are
+template <class FS, class MS, typename O, bool OBJS, bool REC>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(EWaves<FS, OBJS>::value)))
+k_any_E(MainArgs<FS, MS> a) {
+  unsigned n;
+  const int64_t t = launch_tile(a, n);
+  if (t >= 0) any_E_tile<FS, MS, O, OBJS, true, REC>(a, (unsigned)t, a.q);
+}
+
+// The tiles that meet an object, one workgroup each.
+template <class FS, class MS, typename O>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(EWaves<FS>::value)))
+k_object_E(MainArgs<FS, MS> a, const uint32_t* tiles) {
+  any_E_tile<FS, MS, O, true, true, false, true>(a, cp(tiles)[blockIdx.x], a.q);
+}
+
+// Main H kernel, general form: the mirror image of the E kernel. Its differences are
 // forward ones, so workgroups take the tiles in decreasing order (the +y/+z
 // neighbour tiles were read just before, by the same XCD) and march along -x,
 // keeping E of plane i+1 in registers.
 template <class FS, class MS, bool NT>
-__device__ __forceinline__ void main_H_tile(const MainArgs<FS, MS>& __restrict__ a, unsigned tile) {
+__device__ __forceinline__ void any_H_tile(const MainArgs<FS, MS>& __restrict__ a, unsigned tile) {
   using T = typename FS::R;
   const Dims d = a.d;
   int j, k, i0, i1;
@@ -936,11 +1281,84 @@ __device__ __forceinline__ void main_H_tile(const MainArgs<FS, MS>& __restrict__
   }
 }
 
+// Main H kernel: the mirror image of the E kernel, marching along -x.
+template <class FS, class MS, bool NT>
+__device__ __forceinline__ void main_H_tile(const MainArgs<FS, MS>& __restrict__ a, unsigned tile) {
+  using T = typename FS::R;
+  const Dims d = a.d;
+  int j, k, i0, i1;
+  bool act;
+  tile_column(a, tile, j, k, i0, i1, act);
+  if (!wave_any(act)) return;
+  const int64_t base = (int64_t)i0 * d.px;  // the offsets count from plane i0
+  const uint32_t pc = (uint32_t)(j * d.nz + k), at = (uint32_t)(i1 - 1 - i0) * (uint32_t)d.px + pc;
+  const uint32_t fstep = (uint32_t)d.px * FS::kCell, mstep = (uint32_t)d.px * MS::kCell;
+  uint32_t fo = at * FS::kCell, mo = at * MS::kCell;
+  const uint32_t dk = k < d.nz - 1 ? FS::kCell : 0, dj = j < d.ny - 1 ? (uint32_t)d.nz * FS::kCell : 0;
+  TilePml<false, T> pml;
+  pml.init(a, i1 - 1, j, k);
+  const T zero = T(0);
+  typename FS::Own enext;  // E of plane i+1
+  typename MS::Own ahead{};
+  if constexpr (MS::kAhead) ahead = a.M.template own<NT>(base, mo);
+  for (int i = i1 - 1; i >= i0; --i) {
+    opaque(fo);
+    if constexpr (MS::kCell == FS::kCell) mo = fo;
+    if (i == i1 - 1) enext = a.G.template own<false>(base, i1 < d.nx ? fo + fstep : fo);
+    const typename FS::Own eown = a.G.template own<false>(base, fo);
+    const typename FS::Duo ek = a.G.template duo<0, 1>(base, fo + dk), ej = a.G.template duo<0, 2>(base, fo + dj);
+    typename MS::Own mat;
+    if constexpr (MS::kAhead) {
+      mat = ahead;
+      if (i > i0) ahead = a.M.template own<NT>(base, mo - mstep);
+    } else {
+      mat = a.M.template own<NT>(base, mo);
+    }
+    const typename FS::Own hown = a.F.template own<NT>(base, fo);
+    pml.load(a, i, pc);
+    const T e0 = FS::template value<0>(eown), e1 = FS::template value<1>(eown), e2 = FS::template value<2>(eown);
+    // forward differences; an absent one contributes nothing (grid.py:42-49)
+    Diffs<T> df;
+    df.zy = dj ? FS::template value<0, 2, 2>(ej) - e2 : zero;
+    df.yz = dk ? FS::template value<0, 1, 1>(ek) - e1 : zero;
+    df.xz = dk ? FS::template value<0, 1, 0>(ek) - e0 : zero;
+    df.zx = i < d.nx - 1 ? FS::template value<2>(enext) - e2 : zero;
+    df.yx = i < d.nx - 1 ? FS::template value<1>(enext) - e1 : zero;
+    df.xy = dj ? FS::template value<0, 2, 0>(ej) - e0 : zero;
+    enext = eown;
+    T h[3] = {FS::template value<0>(hown), FS::template value<1>(hown), FS::template value<2>(hown)};
+    T m[3], curl[3], kc[3];
+    a.M.values(mat, m);
+    curl[0] = (zero + df.zy) - df.yz;
+    curl[1] = (zero + df.xz) - df.zx;
+    curl[2] = (zero + df.yx) - df.xy;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      kc[c] = a.sc * m[c];
+      h[c] = h[c] - kc[c] * curl[c];
+    }
+    // objects leave H unchanged (objects.py:131-137, 223-229, 271-277)
+    pml.apply(a, df.zx, df.yx, df.zy, df.xy, df.yz, df.xz, kc, h);
+    opaque(fo);
+    a.F.template put_own<NT>(base, fo, h);
+    fo -= fstep;
+    mo -= mstep;
+    pml.next_plane();
+  }
+}
+
 template <class FS, class MS, bool NT>
 __global__ void __launch_bounds__(1024) k_main_H(MainArgs<FS, MS> a) {
   unsigned n;
   const int64_t t = launch_tile(a, n);
   if (t >= 0) main_H_tile<FS, MS, NT>(a, n - 1 - (unsigned)t);
+}
+
+template <class FS, class MS>
+__global__ void __launch_bounds__(1024) k_any_H(MainArgs<FS, MS> a) {
+  unsigned n;
+  const int64_t t = launch_tile(a, n);
+  if (t >= 0) any_H_tile<FS, MS, true>(a, n - 1 - (unsigned)t);
 }
 
 // ------------------------------------------------------------ batched kernels
@@ -987,6 +1405,10 @@ __device__ __forceinline__ int64_t batch_cyclic_tile(const MainArgs<FS, MS>& a, 
   return c >= 0 && c < (int)nch ? (int64_t)c * per + k % per : -1;
 }
 
+// Form of a batched E launch: the main one, or the general one without and
+// with objects.
+enum { kMainForm, kGeneral, kObjects };
+
 // One position of a batched E launch. The position and its grid are the
 // same for the whole workgroup: say so, so that the grid's arguments are read
 // with scalar loads (and, through the restrict reference of the tile body,
@@ -994,7 +1416,7 @@ __device__ __forceinline__ int64_t batch_cyclic_tile(const MainArgs<FS, MS>& a, 
 // taken by reference, the pointers read from them lost their global address
 // space, and the face tables were read with vector (flat) loads, each cell's
 // face loop waiting on memory (twice the time per launch).
-template <class FS, class MS, typename O, bool OBJS, bool NT>
+template <class FS, class MS, typename O, bool NT, int FORM>
 __device__ __forceinline__ void batch_E_at(BatchArgs<FS, MS> b, int64_t it, int64_t q) {
   const int64_t u = __builtin_amdgcn_readfirstlane((int)it);
   const int s = __builtin_amdgcn_readfirstlane(gp(b.item_sim)[u]);
@@ -1003,13 +1425,14 @@ __device__ __forceinline__ void batch_E_at(BatchArgs<FS, MS> b, int64_t it, int6
     t = batch_cyclic_tile(b.sims[s], (unsigned)t, b.rot[s]);
     if (t < 0) return;
   }
-  main_E_tile<FS, MS, O, OBJS, NT>(b.sims[s], (unsigned)t, q);
+  if constexpr (FORM == kMainForm) main_E_tile<FS, MS, false, NT>(b.sims[s], (unsigned)t, q);
+  else any_E_tile<FS, MS, O, FORM == kObjects, NT>(b.sims[s], (unsigned)t, q);
 }
 
 // One position of a batched H launch: each grid's tiles in decreasing order
 // (the mirror of the E kernel's order, as for one grid; contiguous dealing
 // walks the whole list from its end).
-template <class FS, class MS, bool NT>
+template <class FS, class MS, bool NT, bool ANY>
 __device__ __forceinline__ void batch_H_at(BatchArgs<FS, MS> b, int64_t it) {
   const int64_t u = __builtin_amdgcn_readfirstlane((int)(b.cyclic ? it : b.total - 1 - it));
   const int s = __builtin_amdgcn_readfirstlane(gp(b.item_sim)[u]);
@@ -1021,34 +1444,35 @@ __device__ __forceinline__ void batch_H_at(BatchArgs<FS, MS> b, int64_t it) {
     if (t < 0) return;
     t = (int64_t)per * nch - 1 - t;
   }
-  main_H_tile<FS, MS, NT>(b.sims[s], (unsigned)t);
+  if constexpr (ANY) any_H_tile<FS, MS, NT>(b.sims[s], (unsigned)t);
+  else main_H_tile<FS, MS, NT>(b.sims[s], (unsigned)t);
 }
 
 // LOOP: a persistent grid of workgroups walking the list; otherwise one
 // position per workgroup, with no loop around the tile body (the loop's
 // live values made the compiler spill scalar registers to vector lanes,
 // ~50 more vector instructions per wavefront).
-template <class FS, class MS, typename O, bool OBJS, bool NT, bool LOOP>
+template <class FS, class MS, typename O, bool NT, bool LOOP, int FORM>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(EWaves<FS>::value)))
 k_batch_E(BatchArgs<FS, MS> b) {
   const int64_t q = *b.q;
   const int64_t it0 = b.cyclic ? (int64_t)blockIdx.x : (int64_t)xcd_tile(blockIdx.x, gridDim.x);
   if constexpr (LOOP) {
-    for (int64_t it = it0; it < b.total; it += gridDim.x) batch_E_at<FS, MS, O, OBJS, NT>(b, it, q);
+    for (int64_t it = it0; it < b.total; it += gridDim.x) batch_E_at<FS, MS, O, NT, FORM>(b, it, q);
   } else if (it0 < b.total) {
-    batch_E_at<FS, MS, O, OBJS, NT>(b, it0, q);
+    batch_E_at<FS, MS, O, NT, FORM>(b, it0, q);
   }
 }
 
 // H half step; one thread advances the time index (nothing else in this
 // kernel reads it, and the E kernel of this step has completed).
-template <class FS, class MS, bool NT, bool LOOP>
+template <class FS, class MS, bool NT, bool LOOP, bool ANY>
 __global__ void __launch_bounds__(1024) k_batch_H(BatchArgs<FS, MS> b) {
   const int64_t it0 = b.cyclic ? (int64_t)blockIdx.x : (int64_t)xcd_tile(blockIdx.x, gridDim.x);
   if constexpr (LOOP) {
-    for (int64_t it = it0; it < b.total; it += gridDim.x) batch_H_at<FS, MS, NT>(b, it);
+    for (int64_t it = it0; it < b.total; it += gridDim.x) batch_H_at<FS, MS, NT, ANY>(b, it);
   } else if (it0 < b.total) {
-    batch_H_at<FS, MS, NT>(b, it0);
+    batch_H_at<FS, MS, NT, ANY>(b, it0);
   }
   // after the work: a branch at the top would keep the compiler from
   // treating the tile loop's values as uniform

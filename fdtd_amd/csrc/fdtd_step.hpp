@@ -29,15 +29,6 @@ __device__ __forceinline__ void lds_barrier() {
 #endif
 }
 
-// Read-only tables: the constant address space, so that uniform reads are
-// scalar loads whatever the kernel stores in between.
-template <typename T>
-using cptr = const __attribute__((address_space(4))) T*;
-template <typename T>
-__device__ __forceinline__ cptr<T> cp(const T* p) {
-  return (cptr<T>)p;
-}
-
 // The CPML face of one side in a whole step: its two psi components. psiE is
 // read from one buffer and written to another (neighbouring workgroups
 // recompute E, and so psiE, on their halo cells from the values before the
@@ -130,29 +121,6 @@ struct StepArgs {
   int64_t wave_cap;
   int64_t q;
   int64_t nE, nH;  // half steps already taken (the detectors' clocks)
-};
-
-// Two psi values of one cell and face, `off` bytes into their arrays.
-template <typename T>
-struct Psi {
-  T p0, p1;
-  __device__ __forceinline__ void load(const void* a0, const void* a1, uint32_t off) {
-    p0 = ld_stream<false>(split_ptr(reinterpret_cast<const T*>(a0), off));
-    p1 = ld_stream<false>(split_ptr(reinterpret_cast<const T*>(a1), off));
-  }
-  __device__ __forceinline__ void store(void* a0, void* a1, uint32_t off) const {
-    st_stream<false>(split_ptr(reinterpret_cast<T*>(a0), off), p0);
-    st_stream<false>(split_ptr(reinterpret_cast<T*>(a1), off), p1);
-  }
-  // psi <- psi b, plus (difference) c where the slab has both of its cells
-  __device__ __forceinline__ void advance(T b, T c, bool inner, T d0, T d1) {
-    p0 = p0 * b;
-    p1 = p1 * b;
-    if (inner) {
-      p0 = p0 + d0 * c;
-      p1 = p1 + d1 * c;
-    }
-  }
 };
 
 // The CPML faces normal to one axis at a cell: the side whose slab holds it

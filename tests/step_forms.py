@@ -65,6 +65,9 @@ FORMS = {
         ("LineDetector", {}, (S(2, 14), 7, 6)), ("LineDetector", {}, (S(3, 13), S(2, 12), S(1, 11))),
         ("BlockDetector", {}, (S(4, 7), S(9, 9), S(2, 11))), POINT], True),
     "many_tiles": ((21, 34, 67), faces(6) + [POINT], True),
+    "complex": ((12, 19, 17), faces(3) + [
+        ("Object", dict(permittivity=2.5 + 0.03j), (S(3, 8), S(3, 9), S(5, 12))),
+        ("AbsorbingObject", dict(permittivity=1.5, conductivity=2e4), (S(7, 10), S(6, 11), S(2, 9))), POINT], False),
 }
 BACKENDS = ("hip.float64", "hip.float32", "hip.float32c")
 RUNS = (4, 1, 3)  # even, single and odd runs, half steps and an edit between them
@@ -108,6 +111,43 @@ def advance(grid):
     return out
 
 
+def traced(fdtd, name, backend, env):
+    """The states of `advance` under the environment `env`, and the grid."""
+    fdtd.set_backend(backend)
+    keep = dict(os.environ)
+    try:
+        os.environ.update(env)
+        grid = build(fdtd, name)
+        return advance(grid), grid
+    finally:
+        os.environ.clear()
+        os.environ.update(keep)
+
+
+def unequal(got, want):
+    return [f"state {i}" for i, (a, b) in enumerate(zip(got, want))
+            if not torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))]
+
+
+# launches of the half steps: x planes a workgroup, tile shape, objects in a
+# launch of their own
+SHAPES = {f"cx{cx}_{tile}_{objs}": {"FDTD_HIP_STEP": "0", "FDTD_HIP_CX": str(cx), "FDTD_HIP_FLAT": flat,
+                                    "FDTD_HIP_OBJECT_TILES": tiles}
+          for cx in (1, 2, 3) for tile, flat in (("flat", "1"), ("rows", "0"))
+          for objs, tiles in (("joint", "0"), ("apart", "1"))}
+
+
+def form_differences(fdtd, name, backend, shapes=tuple(SHAPES)):
+    """Launch shapes at which the main form of the half-step kernels differs
+    from the general one."""
+    want, _ = traced(fdtd, name, backend, {"FDTD_HIP_STEP": "0", "FDTD_HIP_GENERAL": "1"})
+    bad = []
+    for shape in shapes:
+        got, _ = traced(fdtd, name, backend, SHAPES[shape])
+        bad += [f"{shape}: {d}" for d in unequal(got, want)]
+    return bad
+
+
 def whole(grid):
     """Whether the grid's plan took whole steps."""
     return isinstance(grid._plan.step_buf, torch.Tensor)
@@ -115,22 +155,9 @@ def whole(grid):
 
 def differences(fdtd, name, backend):
     """Names of what is wrong: differing states, or the other route taken."""
-    fdtd.set_backend(backend)
-    keep = os.environ.get("FDTD_HIP_STEP")
-    try:
-        os.environ["FDTD_HIP_STEP"] = "0"
-        half = build(fdtd, name)
-        want = advance(half)
-        os.environ["FDTD_HIP_STEP"] = "1"
-        grid = build(fdtd, name)
-        got = advance(grid)
-    finally:
-        if keep is None:
-            os.environ.pop("FDTD_HIP_STEP", None)
-        else:
-            os.environ["FDTD_HIP_STEP"] = keep
-    bad = [f"state {i}" for i, (a, b) in enumerate(zip(got, want))
-           if not torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))]
+    want, half = traced(fdtd, name, backend, {"FDTD_HIP_STEP": "0"})
+    got, grid = traced(fdtd, name, backend, {"FDTD_HIP_STEP": "1"})
+    bad = unequal(got, want)
     if whole(half):
         bad.append("half steps were asked for")
     if whole(grid) != FORMS[name][2]:
