@@ -316,6 +316,14 @@ int face_order(const FdtdPlan* p, size_t n_faces) {
   return -1;
 }
 
+// What the kernels need of a's launch shape, once block and chunk are set.
+template <class A>
+void set_divisions(A& a) {
+  a.per = make_divide(plane_tiles(a.d, a.bz_shift, a.by, a.flat));
+  a.row = make_divide((uint32_t)(a.flat ? a.d.nz : (a.d.nz + (1 << a.bz_shift) - 1) >> a.bz_shift));
+  a.nchunks = (uint32_t)((a.d.nx + a.cx - 1) / a.cx);
+}
+
 template <class FS, class MS>
 MainArgs<FS, MS> main_args(const FdtdPlan* p, bool is_H) {
   MainArgs<FS, MS> a{};
@@ -337,6 +345,7 @@ MainArgs<FS, MS> main_args(const FdtdPlan* p, bool is_H) {
   a.by = std::max(1, p->block_threads >> bzs);
   a.cyclic = p->cyclic;
   a.flat = p->flat ? p->block_threads : 0;
+  set_divisions(a);
   a.npts = 0;
   return a;
 }
@@ -390,8 +399,7 @@ unsigned block_of(const MainArgs<FS, MS>& a) {
 
 template <class FS, class MS, typename O>
 void launch_main(const FdtdPlan* p, const MainArgs<FS, MS>& a, bool is_H, hipStream_t st) {
-  const unsigned tiles = plane_tiles(p->d, a.bz_shift, a.by, a.flat);
-  const unsigned nchunks = (unsigned)((p->d.nx + a.cx - 1) / a.cx);
+  const unsigned tiles = a.per.d, nchunks = a.nchunks;
   // x-chunks dealt cyclically to the 8 XCDs (xcd_chunk_tile): whole rounds of 8
   const dim3 grid(tiles * (a.cyclic ? (nchunks + 7) / 8 * 8 : nchunks)), block(block_of(a));
   const bool main = main_form(a);
@@ -797,6 +805,11 @@ int launch_step(FdtdPlan* p, bool back, int64_t q, hipStream_t st) {
     a.ntx = t.ntx;
     a.nty = t.nty;
     a.ntz = t.ntz;
+    a.tiles_yz = make_divide((uint32_t)(t.nty * t.ntz));
+    a.tiles_z = make_divide((uint32_t)t.ntz);
+    a.cells_yz = make_divide((uint32_t)(t.ty * t.tz));
+    a.cells_z = make_divide((uint32_t)t.tz);
+    a.cells_y = make_divide((uint32_t)t.ty);
     const dim3 g((unsigned)(t.ntx * t.nty * t.ntz)), b(kStepThreads);
     if (a.nobjs)
       hipLaunchKernelGGL((k_step<FS, MS, O, true>), g, b, 0, st, a);
@@ -1073,6 +1086,7 @@ void batch_tables(const std::vector<FdtdPlan*>& plans, int block_threads, int cx
       a->cx = std::max(1, std::min(cx, p->d.nx));
       a->by = std::max(1, block_threads >> bzs);
       a->flat = p->flat ? block_threads : 0;
+      set_divisions(*a);
     }
     if (p->fold_points) {
       fold_points(p, aE);

@@ -113,6 +113,7 @@ struct StepArgs {
   const ObjDev* objs;
   int32_t nobjs;
   int32_t tx, ty, tz, ntx, nty, ntz;  // own cells of a tile, tiles along each axis
+  Divide tiles_yz, tiles_z, cells_yz, cells_z, cells_y;  // by nty * ntz, ntz, ty * tz, tz, ty
   int32_t nsrc, ndet;
   int32_t folded;  // point sources join the E update before it is stored
   const StepSrc* srcs;
@@ -184,9 +185,10 @@ __global__ void __launch_bounds__(kStepThreads) k_step(StepArgs<FS, MS> a) {
   FDTD_LDS __align__(16) unsigned char lds_bytes[3 * kStepThreads * sizeof(T)];
   T(*const lds)[kStepThreads] = reinterpret_cast<T(*)[kStepThreads]>(lds_bytes);
   const Dims d = a.d;
-  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x), per = (unsigned)(a.nty * a.ntz);
-  const int i0 = (int)(tile / per) * a.tx, j0 = (int)(tile % per / (unsigned)a.ntz) * a.ty,
-            k0 = (int)(tile % (unsigned)a.ntz) * a.tz;
+  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
+  const unsigned nx = a.tiles_yz.of(tile), nxy = a.tiles_z.of(tile);  // x slabs and z rows of tiles before this one
+  const int i0 = (int)nx * a.tx, j0 = (int)(nxy - nx * (unsigned)a.nty) * a.ty,
+            k0 = (int)(tile - nxy * (unsigned)a.ntz) * a.tz;
   // this work-item's cell: the tile's own cells z fastest, then the halo cells
   // past its last x plane, y row and z column
   const int tid = (int)threadIdx.x, tx = a.tx, ty = a.ty, tz = a.tz, yz = ty * tz;
@@ -195,16 +197,16 @@ __global__ void __launch_bounds__(kStepThreads) k_step(StepArgs<FS, MS> a) {
             end = bz + (a.ntz > 1 ? tx * ty : 0);
   int ii = 0, jj = 0, kk = 0;
   if (tid < by) {
-    ii = tid / yz;
+    ii = (int)a.cells_yz.of(tid);
     const int r = tid - ii * yz;
-    jj = r / tz;
+    jj = (int)a.cells_z.of(r);
     kk = r - jj * tz;
   } else if (tid < bz) {
-    ii = (tid - by) / tz;
+    ii = (int)a.cells_z.of(tid - by);
     jj = ty;
     kk = tid - by - ii * tz;
   } else if (tid < end) {
-    ii = (tid - bz) / ty;
+    ii = (int)a.cells_y.of(tid - bz);
     jj = tid - bz - ii * ty;
     kk = tz;
   }
