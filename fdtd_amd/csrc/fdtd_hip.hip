@@ -120,6 +120,8 @@ struct FdtdPlan {
   int cx = 1;                // x planes per workgroup of the main kernels
   int block_threads = 256;   // threads per workgroup of the main kernels
   bool fold_points = false;  // point sources added inside the E kernel
+  bool srcs_apart = false;   // no cell twice in the sources' lists
+  bool tail_apart = false;   // ... and no source's cell in a detector's list
   bool nontemporal = true;   // read-once streams marked non-temporal
   bool cyclic = false;       // x-chunks dealt cyclically to the XCDs (large grids)
   bool flat = false;         // flat tiles: block_threads consecutive cells of the (y, z) plane
@@ -447,6 +449,56 @@ void fold_points(const FdtdPlan* p, MainArgs<FS, MS>& a) {
   a.wave_cap = p->wave_cap;
 }
 
+// The tail of a half step. Lists of up to kTailCells cells go to one workgroup
+// (a launch of several is no faster for them). Longer ones are spread over the
+// chip, sources and reads in one launch where no cell occurs in two lists. Else
+// the reads are a launch of their own, from the length on where one workgroup
+// takes longer than that launch, and sources that share a cell keep one
+// workgroup. Current detectors and records read cells that are in no list, so
+// after sources they are taken to share cells with them.
+constexpr int64_t kTailCells = 512, kTailSplit = 4096;
+
+template <class FS>
+void launch_tail(const FdtdPlan* p, const TailArgs<FS>& t, bool any_src, hipStream_t st) {
+  int64_t src = 0, reads = t.rec ? 3 * box_cells(t.rb) : 0;
+  for (int i = 0; i < t.nsrc; ++i)
+    if (!t.is_H || p->srcs[i].kind == FDTD_SRC_PLANE) src = std::max(src, (int64_t)p->srcs[i].cells.size());
+  for (const DetHost& d : p->dets) reads = std::max(reads, 3 * (int64_t)d.cells.size());
+  const bool cur = t.is_H && t.ncur > 0;
+  if (cur)
+    for (const CurHost& c : p->curs) reads = std::max(reads, (int64_t)c.pts.size() / 3);
+  auto run = [&](const TailArgs<FS>& a, int64_t n) {
+    const int64_t blocks = n <= kTailCells ? 1 : std::min<int64_t>((n + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_tail<FS>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+  };
+  const int64_t n = std::max(src, reads);
+  if (!any_src || (p->tail_apart && !cur && !t.rec)) return run(t, n);
+  if (n <= kTailSplit) return run(t, 0);
+  TailArgs<FS> a = t;
+  a.ndet = a.ncur = 0;
+  a.rec = nullptr;
+  run(a, p->srcs_apart ? src : 0);
+  if (!t.ndet && !cur && !t.rec) return;
+  a = t;
+  a.nsrc = 0;
+  run(a, reads);
+}
+
+// Whether no cell occurs twice in the sources' lists, and whether no detector
+// samples one of their cells: which lists the tail may spread over workgroups.
+void find_apart(FdtdPlan* p) {
+  p->srcs_apart = p->tail_apart = true;
+  if (p->srcs.empty()) return;
+  std::vector<bool> seen((size_t)p->d.cs);
+  for (const SrcHost& s : p->srcs)
+    for (const int64_t c : s.cells) {
+      if (seen[(size_t)c]) p->srcs_apart = p->tail_apart = false;
+      seen[(size_t)c] = true;
+    }
+  for (const DetHost& d : p->dets)
+    for (const int64_t c : d.cells) p->tail_apart = p->tail_apart && !seen[(size_t)c];
+}
+
 template <class FS, class MS, typename O>
 int launch_half(FdtdPlan* p, bool is_H, int64_t q, hipStream_t st) {
   MainArgs<FS, MS> a = main_args<FS, MS>(p, is_H);
@@ -504,7 +556,7 @@ int launch_half(FdtdPlan* p, bool is_H, int64_t q, hipStream_t st) {
     t.counter_H = p->nH;
     t.ncur = (int32_t)p->curs.size();
     t.curs = p->d_curs;
-    hipLaunchKernelGGL(k_tail<FS>, dim3(1), dim3(256), 0, st, t);
+    launch_tail(p, t, any_src, st);
   }
   FDTD_HIP(hipGetLastError());
   if (is_H) {
@@ -1587,6 +1639,7 @@ int fdtd_plan_finalize(FdtdPlan* p) {
   }
   // point sources fold into the E kernel when nothing runs between the main
   // kernel and the sources (no periodic or staged face) and no detector samples
+  find_apart(p);
   p->fold_points = !p->srcs.empty() && (int)p->srcs.size() <= FOLDED_POINTS && p->dets.empty() && p->curs.empty();
   for (const SrcHost& s : p->srcs) p->fold_points = p->fold_points && s.kind == FDTD_SRC_POINT;
   for (const Bnd& b : p->order) p->fold_points = p->fold_points && !b.periodic;

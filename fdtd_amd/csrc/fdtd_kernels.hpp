@@ -31,7 +31,7 @@
 //   k_face               one CPML face over its slab, for faces registered
 //                        after a periodic boundary (order matters there).
 //   k_periodic           plane copy of a periodic boundary.
-//   k_tail               one workgroup: sources (in order) then detectors.
+//   k_tail               sources (in order) then detectors.
 //   k_batch_E / k_batch_H  the main kernels' tile bodies over the tiles of
 //                        many grids (one launch per half step); k_set_time
 //                        sets their device time index.
@@ -1581,14 +1581,18 @@ struct TailArgs {
   Box rb;
 };
 
-// Sources in registration order, then detector samples; one workgroup so the
-// ordering between sources touching the same cell and the detector reads is
-// kept by workgroup barriers.
+// Sources in registration order, then detector samples. One workgroup keeps
+// the order between sources touching the same cell and the detector reads with
+// its barriers; several workgroups are launched over lists of which no two
+// share a cell (launch_tail), each list spread over all of them. Bound by the
+// chain of loads cell index -> field -> store: in one workgroup a plane source
+// and a plane monitor of ~14000 cells took 26 us a half step at 201x150x97,
+// spread 5.0 us.
 template <class FS>
 __global__ void __launch_bounds__(256) k_tail(TailArgs<FS> a) {
   using T = typename FS::R;
   using Sample = typename FS::Sample;
-  const int tid = threadIdx.x;
+  const int tid = (int)(blockIdx.x * blockDim.x + threadIdx.x), stride = (int)(gridDim.x * blockDim.x);
   for (int s = 0; s < a.nsrc; ++s) {
     const SrcDev& src = a.srcs[s];
     if (a.is_H && src.kind != FDTD_SRC_PLANE) continue;
@@ -1612,7 +1616,7 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs<FS> a) {
       __syncthreads();
       continue;
     }
-    for (int p = tid; p < src.n; p += blockDim.x) {
+    for (int p = tid; p < src.n; p += stride) {
       const int64_t cell = base + gp(src.cells)[p];
       if (src.kind == FDTD_SRC_POINT)
         a.F.put(cell, a.F.get(cell) + w);
@@ -1629,7 +1633,7 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs<FS> a) {
       const CurDev& cd = a.curs[t];
       Sample* const buf = reinterpret_cast<Sample*>(cd.buf) + (a.counter - cd.slot0) * cd.n;
       const T dx = (T)cd.spacing;
-      for (int p = tid; p < cd.n; p += blockDim.x) {
+      for (int p = tid; p < cd.n; p += stride) {
         const int px = gp(cd.pts)[p], py = gp(cd.pts)[cd.n + p], pz = gp(cd.pts)[2 * cd.n + p];
         auto H = [&](int c, int x, int y, int z) {
           x = x < 0 ? x + a.d.nx : x;
@@ -1649,7 +1653,7 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs<FS> a) {
   }
   if (a.rec) {
     const int64_t nr = box_cells(a.rb);
-    for (int64_t p = tid; p < 3 * nr; p += blockDim.x) {
+    for (int64_t p = tid; p < 3 * nr; p += stride) {
       const int c = (int)(p / nr);
       a.rec[p] = a.F.get(c * a.d.cs + box_cell(a.rb, a.d, p - c * nr));
     }
@@ -1658,7 +1662,7 @@ __global__ void __launch_bounds__(256) k_tail(TailArgs<FS> a) {
     const DetDev& det = a.dets[t];
     const int64_t slot = a.counter - (a.is_H ? det.slot0H : det.slot0E);
     Sample* const buf = reinterpret_cast<Sample*>(a.is_H ? det.bufH : det.bufE) + slot * det.n * 3;
-    for (int p = tid; p < det.n * 3; p += blockDim.x) {
+    for (int p = tid; p < det.n * 3; p += stride) {
       const int c = p % 3;
       st_stream<false>(buf + p, a.F.sample(c * a.d.cs + gp(det.cells)[p / 3]));
     }

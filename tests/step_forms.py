@@ -64,6 +64,20 @@ FORMS = {
     "detectors": ((17, 15, 14), faces(3) + [
         ("LineDetector", {}, (S(2, 14), 7, 6)), ("LineDetector", {}, (S(3, 13), S(2, 12), S(1, 11))),
         ("BlockDetector", {}, (S(4, 7), S(9, 9), S(2, 11))), POINT], True),
+    # lists that the half steps' tail spreads over workgroups: in one launch,
+    # the reads in a launch of their own, sources that share cells
+    "wide_apart": ((6, 48, 41), faces(2, (1, 2)) + [
+        ("PlaneSource", dict(period=15, polarization="z"), (2, S(1, 46), S(1, 40))),
+        ("BlockDetector", {}, (S(4, 4), S(1, 45), S(1, 38)))], True),
+    "wide_read_sources": ((6, 48, 41), faces(2, (1, 2)) + [
+        ("PlaneSource", dict(period=15, polarization="y"), (2, S(1, 46), S(1, 40))),
+        ("LineSource", dict(period=11), (4, S(3, 42), 7)),
+        ("BlockDetector", {}, (S(2, 4), S(1, 45), S(1, 38)))], True),
+    "wide_shared": ((6, 48, 41), faces(2, (1, 2)) + [
+        ("PlaneSource", dict(period=15, polarization="y"), (2, S(1, 46), S(1, 40))),
+        ("PlaneSource", dict(period=13, polarization="x"), (S(1, 5), 20, S(1, 40))),
+        ("LineSource", dict(period=11), (2, S(3, 42), 7)),
+        ("BlockDetector", {}, (S(1, 4), S(1, 45), S(1, 38)))], True),
     "many_tiles": ((21, 34, 67), faces(6) + [POINT], True),
     "complex": ((12, 19, 17), faces(3) + [
         ("Object", dict(permittivity=2.5 + 0.03j), (S(3, 8), S(3, 9), S(5, 12))),
