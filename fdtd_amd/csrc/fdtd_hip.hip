@@ -506,9 +506,17 @@ int launch_half(FdtdPlan* p, bool is_H, int64_t q, hipStream_t st) {
     fold_points(p, a);
     a.q = q;
   }
+  // the recording E kernel stores the field too where nothing follows it in
+  // the half step (a gradient at 128x128x64 with a point source, 200 steps:
+  // 16.45 -> 14.74 ms, a launch of 5.4 us and its gap a step)
+  const bool rec_in_main = p->rec_curl && p->rec_plane && p->stages.empty() && (p->fold_points || p->srcs.empty());
   if (!is_H && p->rec_curl) {
     a.rec = reinterpret_cast<typename FS::R*>(p->rec_curl);
     a.rb = p->rec_db;
+    if (rec_in_main) {
+      a.rec_E = reinterpret_cast<typename FS::R*>(p->rec_plane);
+      a.rbE = p->rec_pb;
+    }
   }
   launch_main<FS, MS, O>(p, a, is_H, st);
   for (const Bnd& b : p->stages) {
@@ -535,7 +543,7 @@ int launch_half(FdtdPlan* p, bool is_H, int64_t q, hipStream_t st) {
   bool any_src = false;
   if (!p->fold_points)
     for (const SrcHost& s : p->srcs) any_src |= (!is_H || s.kind == FDTD_SRC_PLANE);
-  const bool rec_plane = !is_H && p->rec_plane;
+  const bool rec_plane = !is_H && p->rec_plane && !rec_in_main;
   if (any_src || !p->dets.empty() || rec_plane || (is_H && !p->curs.empty())) {
     TailArgs<FS> t{};
     t.d = p->d;
@@ -982,7 +990,9 @@ AdjArgs<T> adj_args(const FdtdAdjoint* a) {
   int cx = a->cx > 0 ? a->cx : p->cx;
   if (const char* env = getenv("FDTD_HIP_ADJ_CX")) cx = atoi(env);
   r.cx = std::max(1, std::min(cx, p->d.nx));
-  r.by = std::max(1, p->block_threads >> bzs);
+  r.by = std::max(1, kAdjThreads >> bzs);
+  r.flat = p->flat ? kAdjThreads : 0;
+  set_divisions(r);
   return r;
 }
 
@@ -1019,19 +1029,29 @@ const AdjSide<T>* adj_sides(const FdtdAdjoint* a, bool is_H, int parity) {
   return reinterpret_cast<const AdjSide<T>*>(a->d_sides) + ((is_H ? 0 : 2) + parity) * 6;
 }
 
+// Whether the transposed half steps may take k_adj_H and k_adj_E: no two slabs
+// of an axis overlap, and a launch's offsets fit 32 bits (FDTD_HIP_ADJ_FULL=0
+// keeps the general forms, to check that both agree).
+template <typename T>
+bool adj_apart(const FdtdPlan* p, const AdjArgs<T>& a) {
+  const char* env = getenv("FDTD_HIP_ADJ_FULL");
+  if (env && atoi(env) == 0) return false;
+  int t[3] = {0, 0, 0};
+  for (const FaceHost& f : p->faces) t[f.axis] += f.t;
+  for (const FaceDev& f : p->h_faces)
+    if ((uint64_t)f.slab * sizeof(T) >= (uint64_t)1 << 32) return false;
+  return t[0] <= p->d.nx && t[1] <= p->d.ny && t[2] <= p->d.nz &&
+         ((uint64_t)a.cx + 2) * (uint64_t)p->d.px * sizeof(T) < (uint64_t)1 << 32;
+}
+
 template <typename T>
 int adjoint_steps(FdtdAdjoint* a, int64_t nsteps, const T* curl, const T* plane, hipStream_t st) {
   const FdtdPlan* p = a->plan;
   const int64_t nd = box_cells(a->db), np = box_cells(a->pb);
   AdjArgs<T> args = adj_args<T>(a);
-  const int bz = 1 << args.bz_shift, by = args.by;
-  const unsigned tiles = (unsigned)(((p->d.nz + bz - 1) / bz) * ((p->d.ny + by - 1) / by));
-  const dim3 grid(tiles * (unsigned)((p->d.nx + args.cx - 1) / args.cx)), block(bz * by);
+  const dim3 grid(args.per.d * args.nchunks), block(args.flat ? args.flat : args.by << args.bz_shift);
   const dim3 ygrid((unsigned)((p->d.cs + 255) / 256));
-  // no thread past the (y, z) edges: k_adj_H without its store guard
-  // (FDTD_HIP_ADJ_FULL=0 keeps the guard, to check that both forms agree)
-  const char* full_env = getenv("FDTD_HIP_ADJ_FULL");
-  const bool full = p->d.nz % bz == 0 && p->d.ny % by == 0 && !(full_env && atoi(full_env) == 0);
+  const bool apart = adj_apart<T>(p, args);
   for (int64_t s = nsteps - 1; s >= 0; --s) {
     // each half step transposed in reverse: hard sources, then the periodic
     // copies (reverse registration order), then the main update
@@ -1039,21 +1059,24 @@ int adjoint_steps(FdtdAdjoint* a, int64_t nsteps, const T* curl, const T* plane,
     args.side = adj_sides<T>(a, true, a->parH);
     adj_mask_hard_sources<T>(p, args.lamH, true, st);
     adj_periodic<T>(p, args.lamH, true, st);
-    if (full)
-      hipLaunchKernelGGL((k_adj_H<T, true>), grid, block, 0, st, args);
+    if (apart)
+      hipLaunchKernelGGL(k_adj_H<T>, grid, block, 0, st, args);
     else
-      hipLaunchKernelGGL((k_adj_H<T, false>), grid, block, 0, st, args);
+      hipLaunchKernelGGL(k_adj_any_H<T>, grid, block, 0, st, args);
     a->parH ^= 1;
     args.curl = curl + s * 3 * nd;
     args.side = adj_sides<T>(a, false, a->parE);
     adj_mask_hard_sources<T>(p, args.lamE, false, st);
     adj_periodic<T>(p, args.lamE, false, st);
-    if (args.ybuf) {
-      hipLaunchKernelGGL(k_adj_Y<T>, ygrid, dim3(256), 0, st, args);
+    if (args.ybuf) hipLaunchKernelGGL(k_adj_Y<T>, ygrid, dim3(256), 0, st, args);
+    if (apart && args.ybuf)
       hipLaunchKernelGGL((k_adj_E<T, true>), grid, block, 0, st, args);
-    } else {
+    else if (apart)
       hipLaunchKernelGGL((k_adj_E<T, false>), grid, block, 0, st, args);
-    }
+    else if (args.ybuf)
+      hipLaunchKernelGGL((k_adj_any_E<T, true>), grid, block, 0, st, args);
+    else
+      hipLaunchKernelGGL((k_adj_any_E<T, false>), grid, block, 0, st, args);
     a->parE ^= 1;
   }
   FDTD_HIP(hipGetLastError());

@@ -925,6 +925,9 @@ struct MainArgs {
   // half step inside box `rb`, (3, cells of rb)
   R* rec;
   Box rb;
+  // and the updated field inside box `rbE` (null: left to the tail)
+  R* rec_E;
+  Box rbE;
 };
 
 // Tiles of one x-chunk: row tiles (bz z-cells by `by` z-rows) or flat tiles
@@ -1066,6 +1069,14 @@ __device__ __forceinline__ void any_E_tile(const MainArgs<FS, MS>& __restrict__ 
       if (a.nfaces) pml_cell<true>(a.faces, a.nfaces, d, i, j, k, df, kc, e);
       for (int s = 0; s < a.npts; ++s)  // sources.py:109, registration order
         if (a.pt_cell[s] == cell) e[2] = e[2] + (T)gp(a.wave)[s * a.wave_cap + q];
+      if (REC && a.rec_E) {
+        const int64_t r = box_index(a.rbE, i, j, k);
+        if (r >= 0) {
+          const int64_t nr = box_cells(a.rbE);
+#pragma unroll
+          for (int c = 0; c < 3; ++c) a.rec_E[c * nr + r] = FS::rounded(e[c]);
+        }
+      }
       a.F.template put3_s<NT>(cell, e);
     }
     if constexpr (!FS::kRecords) {
@@ -1739,13 +1750,17 @@ struct AdjArgs {
   double* grad;          // (3, cells of db)
   Box pb;                // objective box: lamE += 2 E
   const T* plane;        // (3, cells of pb) recorded for this step
-  int32_t bz_shift, cx, by;  // launch shape, as for the main kernels
+  int32_t bz_shift, cx, by, flat;  // launch shape, as for the main kernels
+  Divide per, row;
+  uint32_t nchunks;
   // anisotropic objects: the plan's object table and a (3, N) buffer of
   // Y = dJ/d(curl H) of the E half step, written by k_adj_Y
   const ObjDev* objs;
   int32_t nobjs;
   T* ybuf;
 };
+
+constexpr int kAdjThreads = 256;
 
 // Slab layout constants of a face normal to AX: the slab is the grid with
 // axis AX shortened to t; `st` is the slab offset of one step along AX.
@@ -1762,7 +1777,7 @@ __device__ __forceinline__ int64_t slab_step(const Dims& d, int t) {
   else return 1;
 }
 
-// The faces normal to AX at one cell of k_adj_H (see there): the face's own
+// The faces normal to AX at one cell of k_adj_any_H (see there): the face's own
 // psi transpose and the difference terms of this cell and of the face cell
 // one step back along AX (which holds the Y values yb0, yb1). The face's
 // axis is a compile-time constant, so components and signs are too. t_lo and
@@ -1810,7 +1825,7 @@ __device__ __forceinline__ void adj_faces_H(const AdjArgs<T>& a, int t_lo, int t
   }
 }
 
-// The faces normal to AX at one cell of k_adj_E (see there): the face's own
+// The faces normal to AX at one cell of k_adj_any_E (see there): the face's own
 // psi transpose and the difference terms of this cell and of the face cell
 // one step ahead along AX. lc0, lc1 are lamE of the face's components C0, C1
 // at this cell, la0, la1 at the cell ahead (already loaded by the caller).
@@ -1883,23 +1898,16 @@ __global__ void __launch_bounds__(256) k_adj_zero(T* lam, const int64_t* cells, 
 // - ([j>=1] Y_z(j-1) - [j<=ny-2] Y_z(j)), and cyclically. The factor dcoef
 // comes from the transpose of the following E half step (k_adj_E leaves it);
 // after the update the objective's 2 E is added inside the objective box.
-// FULL: the tiles cover the (y, z) plane exactly (no thread past an edge), so
-// the stores need no guard; with a guard, the branch's untaken side leaves
-// the plane's loads unconsumed, and the wait inserted for the next plane's
-// register reuse then also waits for this plane's stores.
-template <typename T, bool FULL>
-__global__ void __launch_bounds__(1024) k_adj_H(AdjArgs<T> a) {
+//
+// General form, for slabs that overlap and planes past 32-bit offsets.
+template <typename T>
+__global__ void __launch_bounds__(kAdjThreads) k_adj_any_H(AdjArgs<T> a) {
   const Dims d = a.d;
-  const int bzs = a.bz_shift, bz = 1 << bzs, by = a.by;
-  const int ntz = (d.nz + bz - 1) >> bzs, nty = (d.ny + by - 1) / by;
-  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int tz = tile % ntz, ty = (tile / ntz) % nty, tx = tile / (ntz * nty);
+  int j, k, i0, i1;
+  bool act;
   // as in the main kernels: every load of a plane at once, threads past the
   // edge on the nearest cell (storing nothing), neighbour offset 0 at an edge
-  const int k0 = tz * bz + (threadIdx.x & (bz - 1)), j0 = ty * by + (threadIdx.x >> bzs);
-  const bool act = FULL || (k0 < d.nz && j0 < d.ny);
-  const int k = min(k0, d.nz - 1), j = min(j0, d.ny - 1);
-  const int i0 = tx * a.cx, i1 = min(i0 + a.cx, d.nx);
+  tile_column(a, xcd_tile(blockIdx.x, gridDim.x), j, k, i0, i1, act);
   const int64_t sy = d.nz, sx = d.px, cs = d.cs;
   const int64_t zm = k > 0 ? 1 : 0, ym = j > 0 ? sy : 0;
   const T zero = T(0), sc = a.sc;
@@ -2044,20 +2052,14 @@ __global__ void __launch_bounds__(256) k_adj_periodic(T* lam, Dims d, int axis, 
   }
 }
 
-// YB: Y read from ybuf (k_adj_Y ran first) instead of gcoef lamE. (A FULL
-// form as for k_adj_H is not used here: without the guard the compiler's
-// register reuse made the float kernel wait for the last plane's stores.)
+// YB: Y read from ybuf (k_adj_Y ran first) instead of gcoef lamE. General form,
+// as for k_adj_any_H.
 template <typename T, bool YB>
-__global__ void __launch_bounds__(1024) k_adj_E(AdjArgs<T> a) {
+__global__ void __launch_bounds__(kAdjThreads) k_adj_any_E(AdjArgs<T> a) {
   const Dims d = a.d;
-  const int bzs = a.bz_shift, bz = 1 << bzs, by = a.by;
-  const int ntz = (d.nz + bz - 1) >> bzs, nty = (d.ny + by - 1) / by;
-  const unsigned tile = gridDim.x - 1 - xcd_tile(blockIdx.x, gridDim.x);
-  const int tz = tile % ntz, ty = (tile / ntz) % nty, tx = tile / (ntz * nty);
-  const int k0 = tz * bz + (threadIdx.x & (bz - 1)), j0 = ty * by + (threadIdx.x >> bzs);
-  const bool act = k0 < d.nz && j0 < d.ny;
-  const int k = min(k0, d.nz - 1), j = min(j0, d.ny - 1);
-  const int i0 = tx * a.cx, i1 = min(i0 + a.cx, d.nx);
+  int j, k, i0, i1;
+  bool act;
+  tile_column(a, gridDim.x - 1 - xcd_tile(blockIdx.x, gridDim.x), j, k, i0, i1, act);
   const int64_t sy = d.nz, sx = d.px, cs = d.cs;
   const int64_t zp = k < d.nz - 1 ? 1 : 0, yp = j < d.ny - 1 ? sy : 0;
   const T zero = T(0), sc = a.sc;
@@ -2070,7 +2072,7 @@ __global__ void __launch_bounds__(1024) k_adj_E(AdjArgs<T> a) {
   int64_t cell = (int64_t)(i1 - 1) * sx + (int64_t)j * sy + k;
   // plane i+1, as loaded: lamE of components 1 and 2 and either their Y
   // (ybuf) or their gcoef (Y = gcoef lamE is formed where it is used, for the
-  // reason given in k_adj_H)
+  // reason given in k_adj_any_H)
   T lz_next = zero, ly_next = zero, fz_next = zero, fy_next = zero;
   if (i1 < d.nx) {
     lz_next = L(2, cell + sx);
@@ -2119,6 +2121,266 @@ __global__ void __launch_bounds__(1024) k_adj_E(AdjArgs<T> a) {
     fy_next = f1;
     lz_next = le2;
     ly_next = le1;
+  }
+}
+
+// The CPML of a transposed half step at one cell, faces normal to one axis,
+// where the slabs of the axis do not overlap: the side whose slab holds the
+// cell, its psi and its neighbour's (one step back along the axis for H, ahead
+// for E; a cell outside the slab has no term of it) and their coefficients.
+template <bool IS_H, typename T>
+struct AdjFace {
+  bool lo = false, hi = false;          // the side
+  bool own = false, near = false;       // the cell's own difference term, its neighbour's
+  uint32_t q = 0, step = 0;             // byte offset in the psi arrays, and a plane further
+  uint32_t qn = 0, l = 0, ln = 0;       // bytes to the neighbour's psi; byte offsets in the profiles
+  double b, c, cn;
+  Psi<T> p, n;
+  // g: place along the axis of dn cells; at(l, t): the cell's place in a slab
+  // of thickness t; st: the slab's cells one step along the axis
+  template <class At>
+  __device__ __forceinline__ void locate(int g, int dn, int tl, int th, uint32_t st, At&& at) {
+    lo = g < tl;
+    hi = g >= dn - th;
+    if (!lo && !hi) return;
+    const int t = lo ? tl : th, at_l = lo ? g : g - (dn - t);
+    own = IS_H ? at_l <= t - 2 : at_l >= 1;
+    near = IS_H ? at_l >= 1 : at_l <= t - 2;
+    q = at(at_l, t) * (uint32_t)sizeof(T);
+    qn = near ? (IS_H ? 0u - st : st) * (uint32_t)sizeof(T) : 0;
+    l = (uint32_t)at_l * (uint32_t)sizeof(double);
+    ln = (uint32_t)(near ? (IS_H ? at_l - 1 : at_l + 1) : at_l) * (uint32_t)sizeof(double);
+  }
+  __device__ __forceinline__ void fetch(cptr<AdjSide<T>> sd) {
+    opaque(q);
+    uint32_t r = q + qn;
+    opaque(r);
+    p.load(sd->pin, sd->pin + sd->slab, q);
+    n.load(sd->pin, sd->pin + sd->slab, r);
+    opaque(l);
+    opaque(ln);
+    b = ld_stream<false>(split_ptr(sd->b, l));
+    c = ld_stream<false>(split_ptr(sd->c, l));
+    cn = ld_stream<false>(split_ptr(sd->c, ln));
+  }
+  __device__ __forceinline__ void load(cptr<AdjSide<T>> sd) {
+    if (lo) fetch(sd);
+    if (hi) fetch(sd + 1);
+  }
+  // v: the updated values of the components 3-AX-C0, 3-AX-C1; y, yn: the
+  // weights of the face's components C0, C1 at the cell and at its neighbour
+  template <int AX>
+  __device__ __forceinline__ void apply(cptr<AdjSide<T>> sd, T y0, T y1, T yn0, T yn1, T v[3]) {
+    constexpr int C0 = AX == 0 ? 1 : 0, C1 = AX == 2 ? 1 : 2;
+    constexpr int S0 = 3 - AX - C0, S1 = 3 - AX - C1;
+    // phi = psi_{C+1} - psi_{C+2} enters H' with a minus sign, E' with a plus sign
+    const T sg0 = (AX == (C0 + 1) % 3) == IS_H ? T(-1) : T(1), sg1 = (AX == (C1 + 1) % 3) == IS_H ? T(-1) : T(1);
+    if (!lo && !hi) return;
+    const T w0 = p.p0 + sg0 * y0, w1 = p.p1 + sg1 * y1;
+    const T bt = (T)b, ct = (T)c, cnt = (T)cn;
+    const Psi<T> out{bt * w0, bt * w1};
+    opaque(q);
+    if (lo) out.store(sd->pout, sd->pout + sd->slab, q);
+    if (hi) out.store((sd + 1)->pout, (sd + 1)->pout + (sd + 1)->slab, q);
+    if (own) {
+      v[S0] = IS_H ? v[S0] - ct * w0 : v[S0] + ct * w0;
+      v[S1] = IS_H ? v[S1] - ct * w1 : v[S1] + ct * w1;
+    }
+    if (near) {
+      const T u0 = n.p0 + sg0 * yn0, u1 = n.p1 + sg1 * yn1;
+      v[S0] = IS_H ? v[S0] + cnt * u0 : v[S0] - cnt * u0;
+      v[S1] = IS_H ? v[S1] + cnt * u1 : v[S1] - cnt * u1;
+    }
+  }
+};
+
+// The three axes of a tile's column.
+template <bool IS_H, typename T>
+struct AdjPml {
+  cptr<AdjSide<T>> sides;
+  int t0, t1;  // thicknesses of the x slabs
+  bool any_x, any_y, any_z;  // the plane is in an x slab; some column of the wavefront in a y (z) slab
+  AdjFace<IS_H, T> x, y, z;
+  __device__ __forceinline__ void init(const AdjArgs<T>& a, int i, int j, int k) {
+    const Dims& d = a.d;
+    sides = cp(a.side);
+    t0 = sides[0].t;
+    t1 = sides[1].t;
+    y.locate(j, d.ny, sides[2].t, sides[3].t, (uint32_t)d.nz, [&](int l, int t) {
+      y.step = (uint32_t)(t * d.nz) * (uint32_t)sizeof(T);
+      return (uint32_t)((i * t + l) * d.nz + k);
+    });
+    z.locate(k, d.nz, sides[4].t, sides[5].t, 1, [&](int l, int t) {
+      z.step = (uint32_t)(t * d.ny) * (uint32_t)sizeof(T);
+      return (uint32_t)((i * d.ny + j) * t + l);
+    });
+    any_y = wave_any(y.lo || y.hi);
+    any_z = wave_any(z.lo || z.hi);
+  }
+  __device__ __forceinline__ void load(const AdjArgs<T>& a, int i, uint32_t pc) {
+    const uint32_t plane = (uint32_t)(a.d.ny * a.d.nz);
+    any_x = i < t0 || i >= a.d.nx - t1;
+    if (any_x) {
+      x.locate(i, a.d.nx, t0, t1, plane, [&](int l, int) { return (uint32_t)l * plane + pc; });
+      x.load(sides);
+    }
+    if (any_y) y.load(sides + 2);
+    if (any_z) z.load(sides + 4);
+  }
+  // to the next plane (H marches up, E down)
+  __device__ __forceinline__ void next_plane() {
+    y.q = IS_H ? y.q + y.step : y.q - y.step;
+    z.q = IS_H ? z.q + z.step : z.q - z.step;
+  }
+};
+
+// The transposed half steps where no slabs overlap: the general forms' sums in
+// their order, with a plane's psi and coefficients loaded with its fields and
+// 32-bit offsets, as in the main kernels (the general forms walk the six sides
+// one after another, each a chain of table, psi and profile loads). Work-items
+// past the plane's edge do the last cell's work in lockstep (main_E_tile).
+// Bound by the memory latency of a plane's one round trip at 4 waves a SIMD (97
+// and 113 registers; held to 5 waves they spill, and take 1.5x the time):
+// 128x128x64 float32 with slabs of 12 cells, E 20.8 -> 18.2 us a launch, H
+// 19.2 -> 17.8. No fewer registers than that in float64: at most 256 threads.
+template <typename T>
+__global__ void __launch_bounds__(kAdjThreads) k_adj_H(AdjArgs<T> a) {
+  const Dims d = a.d;
+  int j, k, i0, i1;
+  bool act;
+  tile_column(a, xcd_tile(blockIdx.x, gridDim.x), j, k, i0, i1, act);
+  if (!wave_any(act)) return;
+  const int ib = max(i0 - 1, 0);  // the offsets count from here
+  const int64_t base = (int64_t)ib * d.px, cs = d.cs;
+  const uint32_t pc = (uint32_t)(j * d.nz + k), step = (uint32_t)d.px * (uint32_t)sizeof(T);
+  uint32_t fo = ((uint32_t)(i0 - ib) * (uint32_t)d.px + pc) * (uint32_t)sizeof(T);
+  const uint32_t dk = k > 0 ? (uint32_t)sizeof(T) : 0, dj = j > 0 ? (uint32_t)d.nz * (uint32_t)sizeof(T) : 0;
+  const T zero = T(0), sc = a.sc;
+  auto ld = [&](const T* p, int c, uint32_t off) { return ld_stream<false>(split_ptr(p + c * cs + base, off)); };
+  AdjPml<true, T> pml;
+  pml.init(a, i0, j, k);
+  T m1p = zero, m2p = zero, l1p = zero, l2p = zero;  // inv_mu and lamH of plane i-1, as loaded
+  for (int i = i0; i < i1; ++i, fo += step, pml.next_plane()) {
+    opaque(fo);
+    if (i == i0) {
+      const uint32_t prev = i > 0 ? fo - step : fo;
+      m1p = ld(a.inv_mu, 1, prev), m2p = ld(a.inv_mu, 2, prev);
+      l1p = ld(a.lamH, 1, prev), l2p = ld(a.lamH, 2, prev);
+    }
+    const T m0 = ld(a.inv_mu, 0, fo), m1 = ld(a.inv_mu, 1, fo), m2 = ld(a.inv_mu, 2, fo);
+    const T l0 = ld(a.lamH, 0, fo), l1 = ld(a.lamH, 1, fo), l2 = ld(a.lamH, 2, fo);
+    const T mk0 = ld(a.inv_mu, 0, fo - dk), mk1 = ld(a.inv_mu, 1, fo - dk);
+    const T lk0 = ld(a.lamH, 0, fo - dk), lk1 = ld(a.lamH, 1, fo - dk);
+    const T mj0 = ld(a.inv_mu, 0, fo - dj), mj2 = ld(a.inv_mu, 2, fo - dj);
+    const T lj0 = ld(a.lamH, 0, fo - dj), lj2 = ld(a.lamH, 2, fo - dj);
+    T e[3] = {ld(a.lamE, 0, fo), ld(a.lamE, 1, fo), ld(a.lamE, 2, fo)};
+    if (a.dcoef) {
+      const T d0 = ld(a.dcoef, 0, fo), d1 = ld(a.dcoef, 1, fo), d2 = ld(a.dcoef, 2, fo);
+      pml.load(a, i, pc);
+      e[0] = d0 * e[0];
+      e[1] = d1 * e[1];
+      e[2] = d2 * e[2];
+    } else {
+      pml.load(a, i, pc);
+    }
+    const T y0 = (sc * m0) * l0, y1 = (sc * m1) * l1, y2 = (sc * m2) * l2;
+    const T yz_prev = (sc * m2p) * l2p, yy_prev = (sc * m1p) * l1p;  // Y at plane i-1
+    const T yy_km = (sc * mk1) * lk1, yx_km = (sc * mk0) * lk0, yz_jm = (sc * mj2) * lj2, yx_jm = (sc * mj0) * lj0;
+    const bool km = k >= 1, kp = k <= d.nz - 2, jm = j >= 1, jp = j <= d.ny - 2, im = i >= 1, ip = i <= d.nx - 2;
+    e[0] = e[0] - (((km ? yy_km : zero) - (kp ? y1 : zero)) - ((jm ? yz_jm : zero) - (jp ? y2 : zero)));
+    e[1] = e[1] - (((im ? yz_prev : zero) - (ip ? y2 : zero)) - ((km ? yx_km : zero) - (kp ? y0 : zero)));
+    e[2] = e[2] - (((jm ? yx_jm : zero) - (jp ? y0 : zero)) - ((im ? yy_prev : zero) - (ip ? y1 : zero)));
+    if (pml.any_x) pml.x.template apply<0>(pml.sides, y1, y2, yy_prev, yz_prev, e);
+    if (pml.any_y) pml.y.template apply<1>(pml.sides + 2, y0, y2, yx_jm, yz_jm, e);
+    if (pml.any_z) pml.z.template apply<2>(pml.sides + 4, y0, y1, yx_km, yy_km, e);
+    const int64_t pp = box_index(a.pb, i, j, k);
+    if (wave_any(pp >= 0) && pp >= 0) {
+      const int64_t np = box_cells(a.pb);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) e[c] = e[c] + T(2) * gp(a.plane)[c * np + pp];
+    }
+    opaque(fo);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) st_stream<false>(split_ptr(a.lamE + c * cs + base, fo), e[c]);
+    m1p = m1, m2p = m2, l1p = l1, l2p = l2;
+  }
+}
+
+template <typename T, bool YB>
+__global__ void __launch_bounds__(kAdjThreads) k_adj_E(AdjArgs<T> a) {
+  const Dims d = a.d;
+  int j, k, i0, i1;
+  bool act;
+  tile_column(a, gridDim.x - 1 - xcd_tile(blockIdx.x, gridDim.x), j, k, i0, i1, act);
+  if (!wave_any(act)) return;
+  const int64_t base = (int64_t)i0 * d.px, cs = d.cs;  // the offsets count from here
+  const uint32_t pc = (uint32_t)(j * d.nz + k), step = (uint32_t)d.px * (uint32_t)sizeof(T);
+  uint32_t fo = ((uint32_t)(i1 - 1 - i0) * (uint32_t)d.px + pc) * (uint32_t)sizeof(T);
+  const uint32_t dk = k < d.nz - 1 ? (uint32_t)sizeof(T) : 0,
+                 dj = j < d.ny - 1 ? (uint32_t)d.nz * (uint32_t)sizeof(T) : 0;
+  const T zero = T(0), sc = a.sc;
+  const T* const fac = YB ? a.ybuf : a.gcoef;  // Y, or gcoef (Y = gcoef lamE)
+  auto ld = [&](const T* p, int c, uint32_t off) { return ld_stream<false>(split_ptr(p + c * cs + base, off)); };
+  auto Y = [&](T f, T l) { return YB ? f : f * l; };
+  AdjPml<false, T> pml;
+  pml.init(a, i1 - 1, j, k);
+  T l1n = zero, l2n = zero, f1n = zero, f2n = zero;  // plane i+1, as loaded
+  for (int i = i1 - 1; i >= i0; --i, fo -= step, pml.next_plane()) {
+    opaque(fo);
+    const uint32_t next = i < d.nx - 1 ? fo + step : fo;
+    if (i == i1 - 1) {
+      l1n = ld(a.lamE, 1, next), l2n = ld(a.lamE, 2, next);
+      f1n = ld(fac, 1, next), f2n = ld(fac, 2, next);
+    }
+    const T l0 = ld(a.lamE, 0, fo), l1 = ld(a.lamE, 1, fo), l2 = ld(a.lamE, 2, fo);
+    const T lk0 = ld(a.lamE, 0, fo + dk), lk1 = ld(a.lamE, 1, fo + dk);
+    const T lj0 = ld(a.lamE, 0, fo + dj), lj2 = ld(a.lamE, 2, fo + dj);
+    const T f0 = ld(fac, 0, fo), f1 = ld(fac, 1, fo), f2 = ld(fac, 2, fo);
+    const T fk0 = ld(fac, 0, fo + dk), fk1 = ld(fac, 1, fo + dk), fj0 = ld(fac, 0, fo + dj), fj2 = ld(fac, 2, fo + dj);
+    T h[3] = {ld(a.lamH, 0, fo), ld(a.lamH, 1, fo), ld(a.lamH, 2, fo)};
+    pml.load(a, i, pc);
+    // the grid's 1/eps where a face weighs lamE with it
+    T g[3] = {zero, zero, zero}, gx1 = zero, gx2 = zero, gy0 = zero, gy2 = zero, gz0 = zero, gz1 = zero;
+    if (pml.any_x || pml.any_y || pml.any_z) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) g[c] = ld(a.inv_eps, c, fo);
+      if (pml.any_x) gx1 = ld(a.inv_eps, 1, next), gx2 = ld(a.inv_eps, 2, next);
+      if (pml.any_y) gy0 = ld(a.inv_eps, 0, fo + dj), gy2 = ld(a.inv_eps, 2, fo + dj);
+      if (pml.any_z) gz0 = ld(a.inv_eps, 0, fo + dk), gz1 = ld(a.inv_eps, 1, fo + dk);
+    }
+    const int64_t pd = box_index(a.db, i, j, k), nd = box_cells(a.db);
+    const bool design = wave_any(pd >= 0);
+    double gr[3] = {0.0, 0.0, 0.0};
+    T cu[3] = {zero, zero, zero};
+    if (design && pd >= 0) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        gr[c] = gp(a.grad)[c * nd + pd];
+        cu[c] = gp(a.curl)[c * nd + pd];
+      }
+    }
+    const T y0 = Y(f0, l0), y1 = Y(f1, l1), y2 = Y(f2, l2);
+    const T yz_next = Y(f2n, l2n), yy_next = Y(f1n, l1n);  // Y at plane i+1
+    const T yy_kp = Y(fk1, lk1), yx_kp = Y(fk0, lk0), yz_jp = Y(fj2, lj2), yx_jp = Y(fj0, lj0);
+    const bool km = k >= 1, kp = k <= d.nz - 2, jm = j >= 1, jp = j <= d.ny - 2, im = i >= 1, ip = i <= d.nx - 2;
+    h[0] = h[0] + (((km ? y1 : zero) - (kp ? yy_kp : zero)) - ((jm ? y2 : zero) - (jp ? yz_jp : zero)));
+    h[1] = h[1] + (((im ? y2 : zero) - (ip ? yz_next : zero)) - ((km ? y0 : zero) - (kp ? yx_kp : zero)));
+    h[2] = h[2] + (((jm ? y0 : zero) - (jp ? yx_jp : zero)) - ((im ? y1 : zero) - (ip ? yy_next : zero)));
+    if (pml.any_x)
+      pml.x.template apply<0>(pml.sides, (sc * g[1]) * l1, (sc * g[2]) * l2, (sc * gx1) * l1n, (sc * gx2) * l2n, h);
+    if (pml.any_y)
+      pml.y.template apply<1>(pml.sides + 2, (sc * g[0]) * l0, (sc * g[2]) * l2, (sc * gy0) * lj0, (sc * gy2) * lj2, h);
+    if (pml.any_z)
+      pml.z.template apply<2>(pml.sides + 4, (sc * g[0]) * l0, (sc * g[1]) * l1, (sc * gz0) * lk0, (sc * gz1) * lk1, h);
+    opaque(fo);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) st_stream<false>(split_ptr(a.lamH + c * cs + base, fo), h[c]);
+    if (design && pd >= 0) {
+      const T le[3] = {l0, l1, l2};
+#pragma unroll
+      for (int c = 0; c < 3; ++c) gp(a.grad)[c * nd + pd] = gr[c] + (double)sc * (double)le[c] * (double)cu[c];
+    }
+    l1n = l1, l2n = l2, f1n = f1, f2n = f2;
   }
 }
 

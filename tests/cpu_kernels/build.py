@@ -24,6 +24,8 @@ OUT_DIR = os.path.join(HERE, "_build")
 OUTPUT = os.path.join(OUT_DIR, "libfdtd_cpu.so")
 WRAPPER = os.path.join(HERE, "fdtd_hip_cpu.cpp")
 SOURCES = [WRAPPER, os.path.join(CSRC, "fdtd_hip.hip"), os.path.join(CSRC, "fdtd_kernels.hpp"),
+           os.path.join(CSRC, "fdtd_step.hpp"),
+           os.path.join(CSRC, "fdtd_step.hpp"),
            os.path.join(INCLUDE, "fdtd_hip.h"), os.path.join(HERE, "hip", "hip_runtime.h"), __file__]
 
 

@@ -15,9 +15,11 @@ import step_forms  # noqa: E402
 
 def main():
     replay.load()
-    for arg in [a for a in sys.argv[1:] if a != "--half"]:
+    for arg in [a for a in sys.argv[1:] if not a.startswith("--")]:
         name, backend = arg.split("/")
         compare = step_forms.form_differences if "--half" in sys.argv else step_forms.differences
+        if "--gradient" in sys.argv:
+            compare = step_forms.gradient_differences
         bad = compare(replay.fdtd, name, backend)
         print(json.dumps({"form": arg, "bad": bad}), flush=True)
 

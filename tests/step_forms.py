@@ -177,3 +177,67 @@ def differences(fdtd, name, backend):
     if whole(grid) != FORMS[name][2]:
         bad.append(f"whole steps: {whole(grid)}")
     return bad
+
+
+# Gradients: the transposed half steps' form for slabs that do not overlap
+# against their general form (FDTD_HIP_ADJ_FULL=0), and the field recorded by
+# the E kernel (up to 4 point sources) against the record of the tail (5).
+GRADIENTS = {
+    # name: (shape, CPML thickness, axes with faces, further objects)
+    "cube": ((17, 18, 19), 4, (0, 1, 2), []),
+    "long_rows": ((9, 7, 71), 2, (0, 1, 2), []),
+    "slabs_meet": ((8, 12, 14), 4, (0, 1, 2), []),
+    "thin_faces": ((11, 10, 23), 1, (0, 1, 2), []),
+    "no_faces": ((9, 8, 7), 0, (), []),
+    "one_axis": ((10, 16, 33), 5, (2,), []),
+    "absorber": ((17, 16, 15), 3, (0, 1, 2), [("AbsorbingObject", dict(permittivity=2.0, conductivity=1e4),
+                                               (S(11, 14), S(3, 12), S(4, 11)))]),
+    "anisotropic": ((17, 16, 15), 3, (1, 2), [("AnisotropicObject", dict(permittivity=2.0),
+                                               (S(11, 14), S(3, 12), S(4, 11)))]),
+}
+ADJOINT_SHAPES = [{"FDTD_HIP_ADJ_CX": str(cx), "FDTD_HIP_FLAT": flat} for cx in (1, 2, 3) for flat in ("1", "0")]
+
+
+def gradient(fdtd, name, sources):
+    from fdtd_amd.adjoint import IntensityGradient
+
+    shape, t, axes, objects = GRADIENTS[name]
+    rng = np.random.RandomState(3)
+    grid = fdtd.Grid(shape, grid_spacing=100e-9, courant_number=0.5,
+                     permittivity=torch.from_numpy(rng.uniform(1.0, 3.0, size=shape + (3,))))
+    for kind, params, key in faces(t, axes) if t else []:
+        grid[key] = fdtd.PML()
+    mid = [n // 2 for n in shape]
+    grid[tuple(mid)] = fdtd.PointSource(period=9, amplitude=0.7)
+    for _ in range(sources - 1):
+        grid[tuple(mid)] = fdtd.PointSource(period=9, amplitude=0.0)
+    box = (S(mid[0] - 3, mid[0] + 1), S(mid[1] - 3, mid[1] + 3), S(mid[2] - 2, mid[2] + 3))
+    perm = torch.from_numpy(rng.uniform(1.0, 3.0, size=(4, 6, 5, 3)))
+    design = fdtd.Object(perm, name="design")
+    grid[box] = design
+    for kind, params, key in objects:
+        grid[key] = getattr(fdtd, kind)(**params)
+    prob = IntensityGradient(grid, design, (mid[0] + 1, S(1, shape[1] - 1), S(2, shape[2] - 1)), 12, checkpoint="record")
+    J, g = prob.gradient(perm)
+    return J, g.clone()
+
+
+def gradient_differences(fdtd, name, backend):
+    fdtd.set_backend(backend)
+    keep = dict(os.environ)
+    out = []
+    try:
+        os.environ.update(ADJOINT_SHAPES[0], FDTD_HIP_ADJ_FULL="0")
+        J, g = gradient(fdtd, name, 5)
+        if not bool(torch.isfinite(g).all()) or float(g.abs().max()) == 0.0:
+            return ["gradient not finite or all zero"]
+        os.environ["FDTD_HIP_ADJ_FULL"] = "1"
+        for env in ADJOINT_SHAPES:
+            os.environ.update(env)
+            J1, g1 = gradient(fdtd, name, 1)
+            if J1 != J or not torch.equal(g, g1):
+                out.append(f"{env}: J {J!r} against {J1!r}, gradient {float((g - g1).abs().max())!r} apart")
+    finally:
+        os.environ.clear()
+        os.environ.update(keep)
+    return out

@@ -46,6 +46,19 @@ def test_main_form_on_the_host():
                     + [f"{n}/{b}" for n in ("flat_z", "objects") for b in step_forms.BACKENDS[1:]], "--half")
 
 
+def test_transposed_forms_on_the_host():
+    run_on_the_host([f"{n}/{b}" for n in step_forms.GRADIENTS for b in step_forms.BACKENDS[:2]], "--gradient")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(step_forms.GRADIENTS))
+@pytest.mark.parametrize("backend", step_forms.BACKENDS[:2])
+def test_transposed_forms_match(name, backend):
+    import fdtd_amd as fdtd
+
+    assert step_forms.gradient_differences(fdtd, name, backend) == []
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,backend", [(n, b) for n in step_forms.FORMS for b in backends(n)])
 def test_whole_steps_match_half_steps(name, backend):
