@@ -142,7 +142,7 @@ struct FdtdPlan {
   // holds a second E, H and psiE; the device tables below belong to the plan
   void* step_ws = nullptr;
   void* step_dev = nullptr;
-  StepSide* d_sides[2] = {nullptr, nullptr};  // E -> second E, and back
+  StepSides sides[2];  // E -> second E, and back
   StepSrc* d_ssrcs = nullptr;
   StepDet* d_sdets = nullptr;
   struct StepTile {
@@ -241,7 +241,6 @@ void free_step(FdtdPlan* p) {
   }
   p->step_dev = nullptr;
   p->step_ws = nullptr;
-  p->d_sides[0] = p->d_sides[1] = nullptr;
   p->d_ssrcs = nullptr;
   p->d_sdets = nullptr;
 }
@@ -738,7 +737,6 @@ int build_step_tables(FdtdPlan* p) {
     off = align_up(off + n);
     return at;
   };
-  const size_t o_f[2] = {take(6 * sizeof(StepSide)), take(6 * sizeof(StepSide))};
   const size_t o_s = take(ns * sizeof(StepSrc)), o_d = take(nd * sizeof(StepDet)), o_b = take((2 + nf) * sizeof(CopySeg));
   std::vector<size_t> o_sc(ns), o_sp(ns), o_dc(nd), o_do(nd);
   for (size_t i = 0; i < ns; ++i) {
@@ -761,18 +759,21 @@ int build_step_tables(FdtdPlan* p) {
   };
   copy_back(ws, p->E, field_bytes(p));
   copy_back(ws + align_up(field_bytes(p)), p->H, field_bytes(p));
+  p->sides[0] = p->sides[1] = StepSides{};
   for (size_t i = 0; i < nf; ++i) {
     const FaceDev& fd = p->h_faces[i];
-    const size_t at = (size_t)(fd.axis * 2 + (fd.high ? 1 : 0)) * sizeof(StepSide);
+    const int at = fd.axis * 2 + (fd.high ? 1 : 0);
     const size_t comp = (size_t)fd.slab * value_bytes(p);
-    char *psiE = static_cast<char*>(fd.psiE), *psiH = static_cast<char*>(fd.psiH);
-    StepSide sd{{psiE, psiE + comp}, {psi2, psi2 + comp}, {psiH, psiH + comp}, fd.bE, fd.cE, fd.bH, fd.cH};
-    std::memcpy(host.data() + o_f[0] + at, &sd, sizeof(sd));
-    for (int c = 0; c < 2; ++c) {
-      sd.psiE_in[c] = psi2 + c * comp;
-      sd.psiE_out[c] = psiE + c * comp;
+    char* const psiE = static_cast<char*>(fd.psiE);
+    for (int back = 0; back < 2; ++back) {
+      StepSides& sd = p->sides[back];
+      sd.psiE_in[at] = back ? psi2 : psiE;
+      sd.psiE_out[at] = back ? psiE : psi2;
+      sd.psiH[at] = fd.psiH;
+      sd.coef[at] = fd.bE;  // cE, bH, cH follow it in the plan's table
+      sd.t[at] = fd.t;
+      sd.slab[at] = (int32_t)fd.slab;
     }
-    std::memcpy(host.data() + o_f[1] + at, &sd, sizeof(sd));
     copy_back(psi2, psiE, 2 * comp);
     psi2 += align_up(2 * (size_t)fd.slab * value_bytes(p));
   }
@@ -817,7 +818,6 @@ int build_step_tables(FdtdPlan* p) {
   step_shape(p, p->step_tile);
   p->step_order = face_order(p, p->faces.size());
   FDTD_HIP(hipMemcpy(p->step_dev, host.data(), total, hipMemcpyHostToDevice));
-  for (int h = 0; h < 2; ++h) p->d_sides[h] = reinterpret_cast<StepSide*>(base + o_f[h]);
   p->d_back = reinterpret_cast<CopySeg*>(base + o_b);
   p->nback = (int)back.size();
   p->d_ssrcs = reinterpret_cast<StepSrc*>(base + o_s);
@@ -843,8 +843,7 @@ int launch_step(FdtdPlan* p, bool back, int64_t q, hipStream_t st) {
     a.H2 = back ? H : H2;
     a.Me = make_mat<MS>(p, false);
     a.Mu = make_mat<MS>(p, true);
-    a.sides = p->d_sides[back ? 1 : 0];
-    for (const FaceHost& f : p->faces) a.t[f.axis * 2 + f.high] = f.t;
+    a.sides = p->sides[back ? 1 : 0];
     a.order = p->step_order;
     a.objs = p->d_objs;
     a.nobjs = (int32_t)p->objs.size();
