@@ -508,11 +508,7 @@ class Grid:
             per = max(2, n // 100)  # whole steps go in pairs
             chunks = [per] * (n // per) + ([n % per] if n % per else [])
         for m in chunks:
-            plan = self._prepare(m, m, m)
-            self._lend_step_workspace(plan)
-            plan.run(self.time_steps_passed, m, self._stream())
-            self._count_halves(m, m)
-            self.time_steps_passed += m
+            self._advance(m)
             if bar is not None:
                 bar.update(m)
         if bar is not None:
@@ -530,10 +526,26 @@ class Grid:
         return bool(flag.item())
 
     def step(self):
-        """E half step, H half step, then advance the time index (grid.py:267-273)."""
-        self.update_E()
-        self.update_H()
-        self.time_steps_passed += 1
+        """E half step, H half step, then advance the time index (grid.py:267-273).
+
+        One library call, a whole step where `run` takes them: two calls of the
+        half steps took 67 against 46-50 us on a 200x200x1 grid, host work."""
+        cls = type(self)
+        if (cls.update_E is not Grid.update_E or cls.update_H is not Grid.update_H
+                or "update_E" in self.__dict__ or "update_H" in self.__dict__):
+            # redefined half steps: honour them
+            self.update_E()
+            self.update_H()
+            self.time_steps_passed += 1
+            return
+        self._advance(1)
+
+    def _advance(self, n):
+        plan = self._prepare(n, n, n)
+        self._lend_step_workspace(plan)
+        plan.run(self.time_steps_passed, n, self._stream())
+        self._count_halves(n, n)
+        self.time_steps_passed += n
 
     def update_E(self):
         """Everything the reference's update_E does, in one fused launch
