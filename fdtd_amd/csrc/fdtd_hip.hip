@@ -1184,6 +1184,7 @@ struct BatchImage {
   std::vector<unsigned char> bytes;
   size_t oE = 0, oH = 0, oF = 0, oR = 0, oQ = 0, oI = 0;
   int64_t total = 0;  // positions of the work list
+  size_t derived = 0;  // of the argument tables: what is derived from the rest of an entry
   bool cyclic = false;
   bool objs = false;
   bool any = false;
@@ -1202,6 +1203,7 @@ int batch_image(const std::vector<FdtdPlan*>& plans, int block_threads, int cx, 
     if (img.total >= (int64_t)1 << 31) return fail(-1, "batch has too many work items");
     img.oE = 0;
     img.oH = align_up(n * sizeof(MA));
+    img.derived = 2 * (align_up(n * sizeof(MA)) - align_up(n * (sizeof(MA) - MA::kDerived)));
     img.oF = img.oH + align_up(n * sizeof(MA));
     img.oR = img.oF + align_up((n + 1) * sizeof(int64_t));
     img.oQ = img.oR + align_up(n * sizeof(int32_t));
@@ -1326,7 +1328,9 @@ BatchTables image_tables(const BatchImage& img, void* base) {
 // the array until the process ends. In host code `scratch` names no device
 // address: the address of the current device's copy comes from
 // hipGetSymbolAddress (static_scratch below), and only that is passed on.
-constexpr size_t kStaticBatchBytes = FDTD_STATIC_BATCH_BYTES;
+// The limit counts an argument without its derived members (MainArgs::kDerived);
+// they take at most as much again, an argument being more than twice them.
+constexpr size_t kStaticBatchTables = FDTD_STATIC_BATCH_BYTES, kStaticBatchBytes = 2 * kStaticBatchTables;
 static __device__ __align__(256) unsigned char scratch[kStaticBatchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -2131,9 +2135,9 @@ int fdtd_batch_run_static(int n, FdtdPlan* const* plans, int block_threads, int 
   if (int rc = select_device(pl[0])) return rc;
   BatchImage img;
   if (int rc = batch_image(pl, block_threads, cx, img)) return rc;
-  if (img.bytes.size() > kStaticBatchBytes)
-    return fail(-6, "the batch's tables need " + std::to_string(img.bytes.size()) + " bytes, more than the " +
-                        std::to_string(kStaticBatchBytes) +
+  if (img.bytes.size() - img.derived > kStaticBatchTables)
+    return fail(-6, "the batch's tables need " + std::to_string(img.bytes.size() - img.derived) + " bytes, more than the " +
+                        std::to_string(kStaticBatchTables) +
                         " of the static tables (FDTD_STATIC_BATCH_BYTES); use fdtd_batch_create for this batch");
   void* base = nullptr;
   if (int rc = static_scratch(pl[0]->device, &base)) return rc;

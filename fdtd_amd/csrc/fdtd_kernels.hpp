@@ -928,6 +928,9 @@ struct MainArgs {
   // and the updated field inside box `rbE` (null: left to the tail)
   R* rec_E;
   Box rbE;
+  // bytes of the members that follow from others: the CPML by side, the folded
+  // points by plane, the divisors
+  static constexpr size_t kDerived = 128;
 };
 
 // Tiles of one x-chunk: row tiles (bz z-cells by `by` z-rows) or flat tiles
