@@ -24,10 +24,11 @@
 //                                    triples
 //
 // Kernels
-//   k_main_E / k_main_H  curl, material update, objects and every CPML face
-//                        registered before the first periodic boundary; a
-//                        workgroup marches along x over a (y,z) tile.
-//                        Memory-bound (~0.16 flop/B).
+//   k_main_E / k_main_H  curl, material update and every CPML face registered
+//                        before the first periodic boundary; a workgroup
+//                        marches along x over a (y,z) tile (~0.16 flop/B).
+//                        k_any_E / k_any_H: the form for any faces, and with
+//                        objects; k_object_E: it over the tiles with objects.
 //   k_face               one CPML face over its slab, for faces registered
 //                        after a periodic boundary (order matters there).
 //   k_periodic           plane copy of a periodic boundary.
