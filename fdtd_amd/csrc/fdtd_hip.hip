@@ -670,16 +670,18 @@ Box cells_box(const FdtdPlan* p, const std::vector<int64_t>& cells) {
 // with the halo cells on which neighbouring workgroups compute the same E
 // (40-60 % of the work-items of a 3D tile, 10-15 % of a 2D one). Up to which
 // size that pays, measured on MI355X against the half steps (us/step, half
-// steps -> whole): 2D 161x97 float64 16.3 -> 5.9, 1400x1400 103 -> 86 (2000 x
-// 2000 173 -> 174); 3D float64 60x52x44 21.0 -> 14.3, 110^3 67.9 -> 60.4 (128^3
-// 92 -> 132); float32 36^3 11.1 -> 7.0, 56^3 12.4 -> 12.0 (72^3 15.1 -> 17.0);
-// compensated 40^3 11.9 -> 8.2, 100^3 42.8 -> 39.5. Complex values take twice the
-// registers and lose from 48^3 on (complex64 from 32^3): half steps only.
+// steps -> whole): 2D 161x97 float64 16.3 -> 5.7, 1000x1000 45.7 -> 31.1 (1400
+// x 1400 77.8 -> 85.9), float32 1400x1400 47.0 -> 40.5; 3D float64 60x52x44 21.0
+// -> 12.7, 100^3 49.4 -> 45.4, with objects 59.0 -> 47.5 (120^3 74.9 -> 108.5);
+// float32 36^3 9.6 -> 6.3, 64^3 13.0 -> 11.3 (72^3 14.9 -> 15.0, 84x80x76 with
+// objects 24.1 -> 24.4); compensated 40^3 11.9 -> 8.2, 100^3 40.7 -> 34.3.
+// Complex values take twice the registers and lose from 48^3 on (complex64 from
+// 32^3): half steps only.
 // FDTD_HIP_STEP: 0 never, 1 whatever the size (the rest of the rule stands).
 bool step_eligible(const FdtdPlan* p) {
   if (is_complex(p)) return false;
   const bool flat = p->d.nx == 1 || p->d.ny == 1 || p->d.nz == 1;
-  const int64_t most = (int64_t)1 << (flat ? 21 : (p->dtype == FDTD_F32 ? 17 : 20));
+  const int64_t most = (int64_t)1 << (p->dtype == FDTD_F32 ? (flat ? 21 : 18) : 20);
   const char* env = getenv("FDTD_HIP_STEP");
   if (env ? atoi(env) == 0 : grid_cells(p) > most) return false;
   if (face_order(p, p->faces.size()) < 0 || p->srcs.size() > 32 || p->dets.size() > 32 || !p->curs.empty()) return false;

@@ -240,15 +240,16 @@ int fdtd_batch_run(FdtdBatch* batch, int64_t q0, int64_t nsteps, void* stream);
  * nsteps is launched directly. */
 int fdtd_batch_run_graph(FdtdBatch* batch, int64_t q0, int64_t nsteps, int64_t steps_per_graph, void* stream);
 
-/* Maximum bytes of batch tables that fdtd_batch_run_static can hold. */
+/* Maximum bytes of batch tables that fdtd_batch_run_static can hold (members
+ * of the per-grid arguments that follow from others are not counted). */
 #define FDTD_STATIC_BATCH_BYTES (4u << 20)
 
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (harnesses that forbid hipMalloc, tight serving loops): the same
  * work as fdtd_batch_create + fdtd_batch_set_launch + fdtd_batch_run over
  * the n finalized plans, and the same results, with the batch's tables
- * (per-grid arguments, work list, time index) kept in a device array of
- * FDTD_STATIC_BATCH_BYTES that the library holds on each GPU it runs on
+ * (per-grid arguments, work list, time index) kept in a device array (of
+ * twice FDTD_STATIC_BATCH_BYTES) that the library holds on each GPU it runs on
  * until the process ends, instead of in memory it allocates. No device
  * memory is allocated or freed. The tables of a launch shape that need more
  * than FDTD_STATIC_BATCH_BYTES are refused (error -6); the 64-grid,

@@ -76,8 +76,8 @@ def test_main_form_matches_general_form(name, backend):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape,backend,taken", [((64, 64, 64), "hip.float64", True), ((64, 64, 64), "hip.float32", False),
-                                                 ((50, 51, 50), "hip.float32", True), ((128, 96, 96), "hip.float64", False),
+@pytest.mark.parametrize("shape,backend,taken", [((64, 64, 64), "hip.float64", True), ((64, 64, 64), "hip.float32", True),
+                                                 ((65, 64, 64), "hip.float32", False), ((1100, 1000, 1), "hip.float64", False), ((128, 96, 96), "hip.float64", False),
                                                  ((1000, 700, 1), "hip.float32", True)])
 def test_size_rule(shape, backend, taken):
     import fdtd_amd as fdtd
