@@ -485,9 +485,13 @@ void launch_tail(const FdtdPlan* p, const TailArgs<FS>& t, bool any_src, hipStre
 
 // Whether no cell occurs twice in the sources' lists, and whether no detector
 // samples one of their cells: which lists the tail may spread over workgroups.
+// Not looked into (a bit per cell of the grid) where every list is short.
 void find_apart(FdtdPlan* p) {
-  p->srcs_apart = p->tail_apart = true;
-  if (p->srcs.empty()) return;
+  int64_t most = 0;
+  for (const SrcHost& s : p->srcs) most = std::max(most, (int64_t)s.cells.size());
+  for (const DetHost& d : p->dets) most = std::max(most, 3 * (int64_t)d.cells.size());
+  p->srcs_apart = p->tail_apart = p->srcs.empty() || most > kTailCells;
+  if (p->srcs.empty() || most <= kTailCells) return;
   std::vector<bool> seen((size_t)p->d.cs);
   for (const SrcHost& s : p->srcs)
     for (const int64_t c : s.cells) {
